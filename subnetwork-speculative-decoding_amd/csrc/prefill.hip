@@ -6,15 +6,19 @@
 // the target's forward over the prompt):
 //
 // * prefill_gemm4_kernel: Y = X W^T over the same packed weights as the decode GEMMs (16 x 32 MFMA
-//   A-operand tiles, any tile grouping) with v_mfma_f32_16x16x32_bf16: one 4-wave workgroup per CU
-//   with a 256 x 256 (o, down, gate/up) or 192 x 256 (q/k/v) output tile, accumulators pinned to the
-//   accumulator registers, operands loaded straight into a five-slot LDS ring, outputs staged through
-//   LDS and stored as 16-byte pieces. The decode epilogues run on the staged tile: SwiGLU for gate/up
-//   (gate / up rows r and r + 8 meet through one v_permlane32_swap), residual add for o and down,
-//   RoPE + KV-cache write for q/k/v; the folded RMSNorm scale comes from a row-scale pass. The launch
-//   is persistent and XCD-aware: the workgroups resident on one XCD sweep blocks of output tiles
-//   together, so the weight and activation tiles they share are fetched into that XCD's L2 once per
-//   block.
+//   A-operand tiles, any tile grouping) with v_mfma_f32_16x16x32_bf16: 4-wave workgroups with output
+//   tiles from 32 x 32 to 256 x 256 chosen by the call's M, N and K (pick_prefill_tile), accumulators
+//   pinned to the accumulator registers, operands loaded straight into LDS rings, outputs staged
+//   through LDS and stored as 16-byte pieces. The decode epilogues run on the staged tile: SwiGLU for
+//   gate/up (gate / up rows r and r + 8 meet through one v_permlane32_swap), residual add for o and
+//   down, RoPE + KV-cache write for q/k/v; the folded RMSNorm scale comes from a row-scale pass. The
+//   launch is persistent and XCD-aware: the workgroups resident on one XCD sweep neighbouring output
+//   tiles together, so the weight and activation tiles they share are fetched into that XCD's L2 once.
+//   4096 rows of the 8B shapes, us (before the memory operations were spread between the MFMAs, the
+//   addresses made scalar and X loaded by whole lines): gate/up 728 (875), down 359 (427), o 111 (132),
+//   q/k/v 183 (227): 0.52 of the MFMA peak at gate/up and down. Taking the loads out of the loop gives
+//   down 230 us: the loads' path through L2 bounds the large tiles; small ones are bound by a step's
+//   chain of barrier, MFMAs and LDS reads.
 // * prefill_attention_kernel: causal flash attention, one wave per (q head, 32 tokens), K/V read
 //   in the cache's 64-slot MFMA-operand blocks; S^T = K Q^T and O^T = V^T P^T on MFMA with the
 //   running max / sum rescaled per 64-key block.
@@ -36,100 +40,134 @@ __device__ __forceinline__ size_t packed_tile(int nb, int kb, int kbt, int group
   return ((size_t)(nb / group) * kbt + kb) * group + nb % group;
 }
 
-// ------------------------------------------------------------------ 4-wave variant
-// One workgroup of 4 waves per CU (one per SIMD) owns a 32 XT (N) x 256 (M) output tile; wave (wn,
-// wm) computes 16 XT x 128 of it (8 XT accumulator tiles, held in the accumulator registers), so
-// with XT = 8 each k-block it reads 16 KiB of operands from LDS for 64 MFMAs -- half the LDS bytes
-// per MFMA of a 64 x 64-per-wave layout, whose LDS reads would match the LDS bandwidth at full MFMA
-// rate. XT = 8 (256 x 256 tiles) serves the plain and SwiGLU projections; q/k/v uses XT = 6
-// (192 x 256 tiles), which at the 8B shape (N 6144) makes 512 tiles, two full rounds of 256 CUs
-// instead of 384 tiles whose second round leaves half the CUs idle. Operands reach LDS by direct
-// global-to-LDS loads (16 bytes per lane, one contiguous KiB per wave instruction: a packed W tile,
-// or 16 tokens x 32 k of X gathered into the MFMA B-operand lane order) into a ring of five k-block
-// slots (all 160 KiB of LDS). Step kb: wait until this wave's loads of k-block kb + 1 have landed
-// (those of kb + 2 and kb + 3 may still run) and pass one barrier; issue the loads of kb + 4 into
-// the slot k-block kb - 1 used; read k-block kb + 1's fragments; run k-block kb's MFMAs on the
-// fragments read one step earlier. The step body takes its LDS slots as restrict pointers, which
-// lets the compiler see that the fragment reads do not touch the slot being loaded (otherwise it
-// waits for every load in flight before each LDS read). The folded RMSNorm's row scales come either
-// from the caller (a row-scale pass) or from sums of squares of the X fragments the waves already
-// hold (wave wn sums fragments 4 wn .. 4 wn + 3 of its 8). Outputs are staged through LDS after the
-// k loop and leave as whole 16-byte pieces: rows of Y (residual read the same way); for q/k/v, rows
-// of q and K-cache slots with RoPE applied on the way out, and 8-slot runs of the V^T cache.
-constexpr int P4_BM = 256, P4_SLOTS = 5, P4_AHEAD = 4;
-constexpr int P4_SLOT_BYTES = 32768;                 // up to 16 W tiles + 16 X tiles of one k-block
-constexpr int P4_ROW = 264;                           // staged output row: up to 256 bf16 + 8 of pad
-constexpr int P4_RN_OFF = P4_BM * P4_ROW * 2;         // norm scales after the staged tile
+// ------------------------------------------------------------------ the GEMM
+// One workgroup of 4 waves owns a 32 XT (N) x 32 YT (M) output tile; wave (wn, wm) computes
+// 16 XT x 16 YT of it, XT YT accumulator tiles held in the accumulator registers. Operands reach LDS
+// by direct global-to-LDS loads, 16 bytes per lane: a packed W tile (one contiguous KiB), or 8 tokens
+// x 64 k of X (eight whole 128-byte lines; the eight 16-byte pieces of token r's line land at
+// positions p ^ (r & 7), so that the fragment reads, 16 tokens x one piece, hit every LDS bank
+// equally). A step is KU k-blocks of 32; W is kept in a ring of P4_WS step slots, X in a ring of XU
+// units of 64 k. Step s: wait until this wave's loads for step s + 1 have landed (those issued in
+// step s - 1 may still run) and pass one barrier; run step s's MFMAs on the fragments read one step
+// earlier, and between them -- a few after every row of MFMAs, so that neither the LDS nor the
+// address unit holds back the next MFMA -- read step s + 1's fragments and issue loads: W of step
+// s + 3, and step s's share of the X unit that replaces the oldest one. Waves' global addresses are
+// scalar pointers plus one 32-bit lane offset, ring positions scalar offsets. The step body takes its
+// LDS areas as restrict pointers, which lets the compiler see that the fragment reads do not touch
+// the areas being loaded (otherwise it waits for every load in flight before each LDS read). Every
+// output element is one chain of MFMAs over k in ascending order whatever the tile shape, so all
+// shapes give the same bits.
 typedef __attribute__((address_space(3))) u32x4_t lds_u32x4;
+typedef __attribute__((address_space(3))) unsigned char lds_byte;
+typedef __attribute__((address_space(3))) void lds_void;
+
+// Sizes of one tile shape. LDS holds the two operand rings during the k loop and the staged output
+// tile (BM rows of ROW bf16) plus the row scales after it.
+template <int EPI, int XT, int YT, int KU, int NS>
+struct P4 {
+  static constexpr int BN = 32 * XT, BM = 32 * YT;
+  static constexpr int LW = XT * KU / 2, LX = YT * KU / 2, PER = LW + LX;  // loads per wave and step
+  static constexpr int WSLOT = 2 * XT * KU * 1024, XUNIT = BM * 128;
+  static constexpr int AHEAD = NS - 1;
+  static constexpr int XU = KU == 1 ? 3 : NS;  // X units: steps of one k-block load half a unit each
+  static constexpr int X_OFF = NS * WSLOT, RING = X_OFF + XU * XUNIT;
+  static constexpr int COLS = EPI == EPI_SWIGLU ? BN / 2 : BN;  // staged columns
+  static constexpr int ROW = COLS + 8;
+  static constexpr int RN_OFF = BM * ROW * 2;
+  static constexpr int STAGE = RN_OFF + BM * 4;
+  static constexpr int LDS = RING > STAGE ? RING : STAGE;
+  static_assert(KU == 2 || (KU == 1 && NS == 4), "an X unit is two k-blocks");
+  static_assert((AHEAD - 1) * PER < 64, "vmcnt");
+  static_assert(XT * KU % 2 == 0 && YT * KU % 2 == 0, "each wave loads whole tiles");
+  static_assert(LDS <= 163840, "160 KiB of LDS");
+};
+
+template <int XT, int YT, int KU>
+struct P4Frag {
+  u32x4_t a[KU][XT], b[KU][YT];
+};
 
 // The k loop's MFMAs are written as inline assembly with the accumulators bound to the accumulator
 // registers ("a"): left to the register allocator, some of the accumulator values land in vector
 // registers and are copied in and out around their MFMAs, which costs up to half the loop's rate
-// depending on the epilogue compiled after it. The first k-block uses srcC = 0 (no read of
-// uninitialised accumulators, no VALU-write-to-MFMA-read hazard); accumulator reuse is 8 XT MFMAs
-// apart, and p4_drain() puts the wait states before the epilogue reads them.
-template <bool INIT>
+// depending on the epilogue compiled after it. The accumulators are zeroed ahead of the first
+// barrier; p4_drain() puts the wait states before the epilogue reads them.
 __device__ __forceinline__ void mfma_acc(f32x4_t& c, const u32x4_t& a, const u32x4_t& b) {
-  if constexpr (INIT) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
-  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
 
-template <int XT>
-__device__ __forceinline__ void p4_drain(f32x4_t (&acc)[XT][8]) {
+template <int XT, int YT>
+__device__ __forceinline__ void p4_drain(f32x4_t (&acc)[XT][YT]) {
   // the epilogue's reads of every accumulator depend on these statements, which follow the wait
   // states (more than the 16x16x32 MFMA's write latency) in program order
   asm volatile("s_nop 15\n\ts_nop 15" : "+a"(acc[0][0]));
 #pragma unroll
   for (int x = 0; x < XT; ++x)
 #pragma unroll
-    for (int y = 0; y < 8; ++y)
+    for (int y = 0; y < YT; ++y)
       if (x | y) asm volatile("" : "+a"(acc[x][y]));
 }
 
-template <bool INIT, int XT>
-__device__ __forceinline__ void p4_step(const u32x4_t* const (&wsrc)[XT / 2], const bf16_t* const (&xsrc)[4],
-                                        size_t woff, size_t xoff, bool issue, lds_u32x4* __restrict__ dA,
-                                        lds_u32x4* __restrict__ dB, const lds_u32x4* __restrict__ nA,
-                                        const lds_u32x4* __restrict__ nB, bool fetch, const u32x4_t (&fa)[XT],
-                                        const u32x4_t (&fb)[8], u32x4_t (&na)[XT], u32x4_t (&nb)[8],
-                                        f32x4_t (&acc)[XT][8], int lane) {
-  if (issue) {
-#pragma unroll
-    for (int r = 0; r < XT / 2; ++r)
-      __builtin_amdgcn_global_load_lds((const void*)(wsrc[r] + woff), (__attribute__((address_space(3))) void*)(dA + r * 64),
-                                       16, 0, 0);
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      __builtin_amdgcn_global_load_lds((const void*)(xsrc[r] + xoff), (__attribute__((address_space(3))) void*)(dB + r * 64),
-                                       16, 0, 0);
+// this wave's loads but the last LATER have landed, then the workgroup barrier (no wait for other
+// memory operations)
+template <int LATER>
+__device__ __forceinline__ void p4_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LATER) : "memory");
+}
+// the same with min(later, N) steps of PER loads still running
+template <int PER, int N>
+__device__ __forceinline__ void p4_wait_steps(int later) {
+  if constexpr (N == 0) {
+    p4_wait<0>();
+  } else {
+    if (later >= N) p4_wait<N * PER>();
+    else p4_wait_steps<PER, N - 1>(later);
   }
-  if (fetch) {
-#pragma unroll
-    for (int y = 0; y < 8; ++y) nb[y] = nB[y * 64 + lane];
-#pragma unroll
-    for (int x = 0; x < XT; ++x) na[x] = nA[x * 64 + lane];
-  }
-#pragma unroll
-  for (int x = 0; x < XT; ++x)
-#pragma unroll
-    for (int y = 0; y < 8; ++y) mfma_acc<INIT>(acc[x][y], fa[x], fb[y]);
 }
 
-// this wave's loads of k-block kb + 1 have landed (the PER = XT / 2 + 4 each of up to `later`
-// later k-blocks may still run), then the workgroup barrier (no wait for other memory operations)
-template <int PER>
-__device__ __forceinline__ void p4_wait(int later) {
-  static_assert(PER == 8 || PER == 7, "XT = 8 or 6");
-  if constexpr (PER == 8) {
-    if (later >= 3) asm volatile("s_waitcnt vmcnt(24)\n\ts_barrier" ::: "memory");
-    else if (later == 2) asm volatile("s_waitcnt vmcnt(16)\n\ts_barrier" ::: "memory");
-    else if (later == 1) asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-  } else {
-    if (later >= 3) asm volatile("s_waitcnt vmcnt(21)\n\ts_barrier" ::: "memory");
-    else if (later == 2) asm volatile("s_waitcnt vmcnt(14)\n\ts_barrier" ::: "memory");
-    else if (later == 1) asm volatile("s_waitcnt vmcnt(7)\n\ts_barrier" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+// Load i of this wave's LW + LX of one step, into its first W tile dW / X piece dX (1 KiB each).
+template <int LW, int LX>
+__device__ __forceinline__ void p4_load(const char* const (&wp)[LW], const char* const (&xp)[LX], uint32_t wlane,
+                                        const uint32_t (&xlane)[LX], int i, lds_byte* dW, lds_byte* dX) {
+  if (i < LW) __builtin_amdgcn_global_load_lds((const void*)(wp[i] + wlane), (lds_void*)(dW + i * 1024), 16, 0, 0);
+  else __builtin_amdgcn_global_load_lds((const void*)(xp[i - LW] + xlane[i - LW]), (lds_void*)(dX + (i - LW) * 1024), 16, 0, 0);
+}
+
+// Read r of this wave's KU (XT + YT) fragments of a step: nW points at its first W tile, nX[u] at its
+// first X tile (16 tokens, 2 KiB apart) for k-block u; lanes already added.
+template <int XT, int YT, int KU>
+__device__ __forceinline__ void p4_fetch(P4Frag<XT, YT, KU>& nf, const lds_byte* nW, const lds_byte* const (&nX)[KU], int r) {
+  const int u = r / (XT + YT), i = r % (XT + YT);
+  if (i < YT) nf.b[u][i] = *(const lds_u32x4*)(nX[u] + i * 2048);
+  else nf.a[u][i - YT] = *(const lds_u32x4*)(nW + (u * 2 * XT + i - YT) * 1024);
+}
+
+// One step: MFMAs on `f`; `nf` <- the next step's fragments; this step's loads into dW / dX.
+template <int XT, int YT, int KU, int LW, int LX>
+__device__ __forceinline__ void p4_step(const char* const (&wp)[LW], const char* const (&xp)[LX], uint32_t wlane,
+                                        const uint32_t (&xlane)[LX], bool load_w, bool load_x, lds_byte* __restrict__ dW,
+                                        lds_byte* __restrict__ dX, const lds_byte* __restrict__ nW,
+                                        const lds_byte* const (&nX)[KU], bool fetch,
+                                        const P4Frag<XT, YT, KU>& f, P4Frag<XT, YT, KU>& nf, f32x4_t (&acc)[XT][YT]) {
+  constexpr int G = KU * XT;             // rows of YT MFMAs
+  constexpr int GM = G > 1 ? G - 1 : 1;  // memory operations follow all but the last row
+  constexpr int R = KU * (XT + YT), L = LW + LX;
+#pragma unroll
+  for (int q = 0; q < G; ++q) {
+    const int u = q / XT, x = q % XT;
+#pragma unroll
+    for (int y = 0; y < YT; ++y) mfma_acc(acc[x][y], f.a[u][x], f.b[u][y]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (q < GM) {
+      if (fetch) {
+#pragma unroll
+        for (int r = R * q / GM; r < R * (q + 1) / GM; ++r) p4_fetch<XT, YT, KU>(nf, nW, nX, r);
+      }
+#pragma unroll
+      for (int i = L * q / GM; i < L * (q + 1) / GM; ++i)
+        if (i < LW ? load_w : load_x) p4_load<LW, LX>(wp, xp, wlane, xlane, i, dW, dX);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
 }
 
@@ -144,20 +182,21 @@ __device__ __forceinline__ float pf_silu(float x) {
 // q/k/v write-out of one staged tile: rows of q and K-cache slots (RoPE applied here), then 8-slot
 // runs of V^T. Staged column 16 t + i holds weight tile nb0 + t's row i: rotary dim p 8 + i
 // (i < 8) or hd / 2 + p 8 + i - 8 (i >= 8) of its head -- both halves of each rotary pair. Thread
-// t's q/k items are (token, weight tile) = divmod(t + 256 i, 2 XT), i < 2 XT; their rotary cos / sin
+// t's q/k items are (token, weight tile) = divmod(t + 256 i, 2 XT), i < NI; their rotary cos / sin
 // pieces are loaded by p4_qkv_rope() before the tile is staged (clamped addresses for items that
 // are not q/k, so the loads are unconditional), so their latency overlaps the staging.
-template <int XT>
+template <class C>
 struct P4Rope {
-  Pack8 cs[2 * XT], sn[2 * XT];
+  static constexpr int NWT = C::BN / 16, ITEMS = C::BM * NWT, NI = (ITEMS + 255) / 256;
+  Pack8 cs[NI], sn[NI];
 };
 
-template <int XT>
-__device__ __forceinline__ void p4_qkv_rope(const GemmArgs& a, int nb0, int m0, int pos0, int t, P4Rope<XT>& r) {
-  constexpr int NWT = 2 * XT;
+template <class C>
+__device__ __forceinline__ void p4_qkv_rope(const GemmArgs& a, int nb0, int m0, int pos0, int t, P4Rope<C>& r) {
+  constexpr int NWT = P4Rope<C>::NWT;
   const int half = a.head_dim >> 1;
 #pragma unroll
-  for (int i = 0; i < NWT; ++i) {
+  for (int i = 0; i < P4Rope<C>::NI; ++i) {
     const int it = t + 256 * i, row = it / NWT, tt = it % NWT;
     const QkvTile q = qkv_tile(a, nb0 + tt);
     const int pos = min(max(pos0 + m0 + row, 0), (int)a.rope_rows - 1);
@@ -167,23 +206,23 @@ __device__ __forceinline__ void p4_qkv_rope(const GemmArgs& a, int nb0, int m0, 
   }
 }
 
-template <int XT>
+template <class C>
 __device__ __forceinline__ void p4_qkv_out(const GemmArgs& a, const bf16_t* stage, int nb0, int m0, int pos0, int t,
-                                           const P4Rope<XT>& r) {
-  constexpr int NWT = 2 * XT;  // weight tiles of the workgroup tile
+                                           const P4Rope<C>& r) {
+  constexpr int NWT = P4Rope<C>::NWT;  // weight tiles of the workgroup tile
   const int hd = a.head_dim, half = hd >> 1;
   const int n_wt = min(NWT, a.N / 16 - nb0);  // N is a multiple of 16 (q/k/v shape)
   const bool qvec = a.ldy % 8 == 0 && ((uintptr_t)a.Y & 15) == 0;
   // q and K: one (token, weight tile) per item, two 16-byte pieces (the pair's halves)
 #pragma unroll
-  for (int i = 0; i < NWT; ++i) {
+  for (int i = 0; i < P4Rope<C>::NI; ++i) {
     const int it = t + 256 * i, row = it / NWT, tt = it % NWT, m = m0 + row;
-    if (tt >= n_wt || m >= a.M) continue;
+    if (it >= P4Rope<C>::ITEMS || tt >= n_wt || m >= a.M) continue;
     const QkvTile q = qkv_tile(a, nb0 + tt);
     if (q.region == 2) continue;
     Pack8 lo, hi, olo, ohi;
-    lo.u = *(const uint4*)(stage + row * P4_ROW + tt * 16);
-    hi.u = *(const uint4*)(stage + row * P4_ROW + tt * 16 + 8);
+    lo.u = *(const uint4*)(stage + row * C::ROW + tt * 16);
+    hi.u = *(const uint4*)(stage + row * C::ROW + tt * 16 + 8);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float xl = bf2f(lo.h[e]), xh = bf2f(hi.h[e]), c = bf2f(r.cs[i].h[e]), s = bf2f(r.sn[i].h[e]);
@@ -211,7 +250,7 @@ __device__ __forceinline__ void p4_qkv_out(const GemmArgs& a, const bf16_t* stag
   }
   // V^T: one (8-slot run, staged column) per item; runs cut by the tile's first or last token, or by
   // M, are written element by element (the neighbouring tile writes the rest of such a run)
-  const int s_lo = pos0 + m0, s_hi = pos0 + min(m0 + P4_BM, a.M);  // slots [s_lo, s_hi)
+  const int s_lo = pos0 + m0, s_hi = pos0 + min(m0 + C::BM, a.M);  // slots [s_lo, s_hi)
   const int g_lo = s_lo >> 3, n_runs = ((s_hi + 7) >> 3) - g_lo;
   for (int it = t; it < n_runs * NWT * 16; it += 256) {
     const int run = it / (NWT * 16), c = it % (NWT * 16), tt = c >> 4, i = c & 15;
@@ -224,113 +263,213 @@ __device__ __forceinline__ void p4_qkv_out(const GemmArgs& a, const bf16_t* stag
     if (s0 >= s_lo && s0 + 8 <= s_hi) {
       Pack8 v;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v.h[e] = stage[(s0 + e - s_lo) * P4_ROW + c];
+      for (int e = 0; e < 8; ++e) v.h[e] = stage[(s0 + e - s_lo) * C::ROW + c];
       *(uint4*)(vt + v_off(s0, d, hd)) = v.u;
     } else {
       for (int e = 0; e < 8; ++e) {
         const int s = s0 + e;
-        if (s >= s_lo && s < s_hi) vt[v_off(s, d, hd)] = stage[(s - s_lo) * P4_ROW + c];
+        if (s >= s_lo && s < s_hi) vt[v_off(s, d, hd)] = stage[(s - s_lo) * C::ROW + c];
       }
     }
   }
 }
 
-template <int EPI, bool RS, int XT>
-__global__ __launch_bounds__(256, 1) void prefill_gemm4_kernel(GemmArgs a, int group, int n_mt, int n_nt, int pos0,
-                                                               int sb_n, int sb_m) {
-  static_assert(XT == 8 || XT == 6, "8 or 6 weight tiles per wave");
-  static_assert(EPI != EPI_SWIGLU || XT == 8, "SwiGLU pairs need whole 16-column output groups");
-  constexpr int WR = XT / 2, PER = WR + 4;  // W tiles each wave loads per k-block; loads per k-block
-  __shared__ __align__(16) unsigned char smem[P4_SLOTS * P4_SLOT_BYTES];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+// OCC: workgroups per CU the registers are budgeted for.
+template <int EPI, bool RS, int XT, int YT, int KU, int NS, int OCC>
+__global__ __launch_bounds__(256, OCC) void prefill_gemm4_kernel(GemmArgs a, int group, int n_mt, int n_nt, int pos0,
+                                                                 int band) {
+  typedef P4<EPI, XT, YT, KU, NS> C;
+  constexpr int LW = C::LW, LX = C::LX, PER = C::PER;
+  __shared__ __align__(16) unsigned char smem[C::LDS];
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int j = lane & 15, g = lane >> 4;
   const int wn = w & 1, wm = w >> 1;
   const int n_rt = (a.N + 127) / 128 * 8;
-  const int kbt = a.kb_total;
-  const u32x4_t* W = (const u32x4_t*)a.W;
-  // slot s: W tiles at s * 32 KiB, X tiles 16 KiB further; tile i is 64 lanes x 16 bytes
-  auto slotA = [&](int kb, int tile) { return (lds_u32x4*)(smem + (kb % P4_SLOTS) * P4_SLOT_BYTES) + tile * 64; };
-  auto slotB = [&](int kb, int tile) {
-    return (lds_u32x4*)(smem + (kb % P4_SLOTS) * P4_SLOT_BYTES + 16384) + tile * 64;
-  };
-  float* rn_s = (float*)(smem + P4_RN_OFF);
-  bf16_t* stage = (bf16_t*)smem;  // [256 tokens][P4_ROW] after the k loop
-  // persistent and XCD-aware: the workgroups resident on one XCD sweep blocks of sb_n x sb_m output
-  // tiles together, so the weight and activation tiles they share are fetched into that XCD's L2
-  // once per block
-  const int xcd = blockIdx.x % 8, jw = blockIdx.x / 8;
-  const int n_bn = (n_nt + sb_n - 1) / sb_n, n_bm = (n_mt + sb_m - 1) / sb_m;
-  for (int blk = xcd; blk < n_bn * n_bm; blk += 8) {
-  const int bn = (blk / n_bm) * sb_n + jw % sb_n, bm = (blk % n_bm) * sb_m + jw / sb_n;
-  if (bn >= n_nt || bm >= n_mt || jw >= sb_n * sb_m) continue;  // uniform per workgroup
-  const int nb0 = bn * 2 * XT, m0 = bm * P4_BM;
-  // wave w loads W tiles WR w .. WR w + WR - 1 and X tiles 4w .. 4w + 3 of every k-block (row tiles
-  // past the weight's last load that one; tokens past M load the last row: neither is stored)
-  const u32x4_t* wsrc[WR];
-  const bf16_t* xsrc[4];
+  const int kbt = a.kb_total, n_steps = kbt / KU;  // kbt is even (K % 64 == 0)
+  float* rn_s = (float*)(smem + C::RN_OFF);
+  bf16_t* stage = (bf16_t*)smem;  // [BM tokens][ROW] after the k loop
+  // Persistent and XCD-aware: output tiles are ordered in bands of `band` row tiles, rows fastest,
+  // and each XCD takes one contiguous run of that order, so the workgroups resident on it work on a
+  // block of neighbouring tiles and fetch the weight and activation tiles they share into that XCD's
+  // L2 once.
+  const int tiles = n_mt * n_nt, xcd = blockIdx.x % 8, per_xcd = (tiles + 7) / 8;
+  for (int it = blockIdx.x / 8; it < per_xcd; it += gridDim.x / 8) {
+  const int tile = xcd * per_xcd + it;
+  if (tile >= tiles) break;  // uniform per workgroup
+  const int bnd = tile / (band * n_nt), in_band = tile - bnd * band * n_nt, hb = min(band, n_mt - bnd * band);
+  const int nb0 = in_band / hb * 2 * XT, m0 = (bnd * band + in_band % hb) * C::BM;
+  // Wave w loads W tiles LW w .. of every slot ([k-block][row tile]; row tiles past the weight's last
+  // load that one) and 8-token pieces of X: with KU = 2, pieces LX w .. of the unit; with KU = 1,
+  // pieces 2 LX w .. + LX - 1 in a unit's first step and the next LX in its second (tokens past M
+  // load the last row: neither is stored).
+  const char *wp[LW], *xp[KU == 1 ? 2 : 1][LX];
+  uint32_t xlane[KU == 1 ? 2 : 1][LX];
 #pragma unroll
-  for (int r = 0; r < WR; ++r) {
-    const int nb = min(nb0 + WR * w + r, n_rt - 1);
-    wsrc[r] = W + packed_tile(nb, 0, kbt, group) * 64 + lane;
+  for (int r = 0; r < LW; ++r) {
+    const int i = LW * w + r, nb = min(nb0 + i % (2 * XT), n_rt - 1);
+    wp[r] = (const char*)a.W + (packed_tile(nb, 0, kbt, group) + (size_t)(i / (2 * XT)) * group) * 1024;
   }
+  const int l8 = lane >> 3;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) xsrc[r] = a.X + (size_t)min(m0 + 16 * (4 * w + r) + j, a.M - 1) * a.ldx + g * 8;
-  const size_t wstep = (size_t)group * 64;
-
-  f32x4_t acc[XT][8];  // written first by k-block 0's srcC = 0 MFMAs
-
-  // prologue: loads of k-blocks 0 .. 3, fragments of k-block 0
-  u32x4_t a0[XT], b0[8], a1[XT], b1[8];
-  for (int p = 0; p < P4_AHEAD; ++p)
-    if (p < kbt) {
+  for (int h = 0; h < (KU == 1 ? 2 : 1); ++h)
 #pragma unroll
-      for (int r = 0; r < WR; ++r)
-        __builtin_amdgcn_global_load_lds((const void*)(wsrc[r] + p * wstep),
-                                         (__attribute__((address_space(3))) void*)(slotA(p, WR * w) + r * 64), 16, 0, 0);
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        __builtin_amdgcn_global_load_lds((const void*)(xsrc[r] + (size_t)p * 32),
-                                         (__attribute__((address_space(3))) void*)(slotB(p, 4 * w) + r * 64), 16, 0, 0);
+    for (int r = 0; r < LX; ++r) {
+      const int row0 = min(m0 + 8 * (KU == 1 ? 2 * LX * w + h * LX + r : LX * w + r), a.M - 1);
+      xp[h][r] = (const char*)(a.X + (size_t)row0 * a.ldx);
+      xlane[h][r] = (uint32_t)(min(row0 + l8, a.M - 1) - row0) * (uint32_t)a.ldx * 2 + ((lane & 7) ^ l8) * 16;
     }
-  // k-block 0 landed (up to three later ones may still run), fragments of 0
-  p4_wait<PER>(min(kbt, P4_AHEAD) - 1);
-#pragma unroll
-  for (int y = 0; y < 8; ++y) b0[y] = slotB(0, wm * 8)[y * 64 + lane];
-#pragma unroll
-  for (int x = 0; x < XT; ++x) a0[x] = slotA(0, wn * XT)[x * 64 + lane];
+  const uint32_t wlane = lane * 16;
+  const size_t wstep = (size_t)group * 1024 * KU;
+  lds_byte* const lds = (lds_byte*)smem;
+  lds_byte* const dw0 = lds + w * LW * 1024;                                        // this wave's load areas
+  lds_byte* const dx0 = lds + C::X_OFF + w * (KU == 1 ? 2 : 1) * LX * 1024;
+  // and fragments: W tiles wn XT .., X tiles wm YT .. (k-block u's piece of token j sits at
+  // position (4 u + g) ^ (j & 7))
+  const lds_byte* const rw0 = lds + wn * XT * 1024 + lane * 16;
+  const lds_byte* const rx0 = lds + C::X_OFF + wm * YT * 2048 + j * 128;
+  const uint32_t px[2] = {(uint32_t)((g ^ (j & 7)) * 16), (uint32_t)(((4 + g) ^ (j & 7)) * 16)};
 
-  auto step = [&](auto init, int kb, const u32x4_t (&fa)[XT], const u32x4_t (&fb)[8], u32x4_t (&na)[XT],
-                  u32x4_t (&nb)[8]) {
-    p4_wait<PER>(min(kbt - 2 - kb, 2));  // loads of kb + 2 .. kb + 3 may still run
-    const int ki = kb + P4_AHEAD;
-    p4_step<decltype(init)::value, XT>(wsrc, xsrc, (size_t)ki * wstep, (size_t)ki * 32, ki < kbt, slotA(ki, WR * w),
-                                       slotB(ki, 4 * w), slotA(kb + 1, wn * XT), slotB(kb + 1, wm * 8), kb + 1 < kbt,
-                                       fa, fb, na, nb, acc, lane);
+  f32x4_t acc[XT][YT];
+#pragma unroll
+  for (int x = 0; x < XT; ++x)
+#pragma unroll
+    for (int y = 0; y < YT; ++y) {
+      acc[x][y] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      asm volatile("" : "+a"(acc[x][y]));  // here, not in each path of the k loop
+    }
+
+  // Prologue: KU = 2: W and X of steps 0 .. 2. KU = 1: X unit 0 and W 0, then what step 0 and step 1
+  // wait for one step's worth of loads after another: W 1, half of unit 1; W 2, its other half.
+  auto load_x_half = [&](int h, uint32_t off) {
+#pragma unroll
+    for (int i = LW; i < PER; ++i)
+      p4_load<LW, LX>(wp, xp[KU == 1 ? h : 0], wlane, xlane[KU == 1 ? h : 0], i, dw0,
+                      dx0 + off + (KU == 1 ? h * LX * 1024 : 0));
   };
-  using first_t = std::integral_constant<bool, true>;
-  using rest_t = std::integral_constant<bool, false>;
-  // kbt is even (K % 64 == 0): step 0, pairs (1, 2) .. (kbt - 3, kbt - 2), step kbt - 1
-  step(first_t{}, 0, a0, b0, a1, b1);
-  for (int kb = 1; kb + 1 < kbt; kb += 2) {
-    step(rest_t{}, kb, a1, b1, a0, b0);
-    step(rest_t{}, kb + 1, a0, b0, a1, b1);
+  auto load_w_step = [&](uint32_t off) {
+#pragma unroll
+    for (int i = 0; i < LW; ++i) p4_load<LW, LX>(wp, xp[0], wlane, xlane[0], i, dw0 + off, dx0);
+#pragma unroll
+    for (int r = 0; r < LW; ++r) wp[r] += wstep;
+  };
+  auto next_unit = [&](int h) {
+#pragma unroll
+    for (int r = 0; r < LX; ++r) xp[KU == 1 ? h : 0][r] += 128;
+  };
+  P4Frag<XT, YT, KU> f0, f1;
+  if constexpr (KU == 1) {
+    load_x_half(0, 0);
+    load_x_half(1, 0);
+    next_unit(0);
+    next_unit(1);
+    load_w_step(0);
+    load_w_step(C::WSLOT);  // kbt is even
+    if (n_steps > 2) {
+      load_x_half(0, C::XUNIT);
+      load_w_step(2 * C::WSLOT);
+      load_x_half(1, C::XUNIT);
+      next_unit(0);
+      next_unit(1);
+    }
+    if (n_steps > 2) p4_wait<2 * PER>();
+    else p4_wait<0>();
+  } else {
+#pragma unroll
+    for (int p = 0; p < C::AHEAD; ++p)
+      if (p < n_steps) {
+        load_w_step(p * C::WSLOT);
+        load_x_half(0, p * C::XUNIT);
+        next_unit(0);
+      }
+    p4_wait_steps<PER, C::AHEAD - 1>(n_steps - 1);
   }
-  step(rest_t{}, kbt - 1, a1, b1, a0, b0);
-  p4_drain<XT>(acc);
+  {
+    const lds_byte* nx[KU];
+#pragma unroll
+    for (int u = 0; u < KU; ++u) nx[u] = rx0 + px[u];
+#pragma unroll
+    for (int r = 0; r < KU * (XT + YT); ++r) p4_fetch<XT, YT, KU>(f0, rw0, nx, r);
+  }
+
+  // ring positions (bytes): W slots of steps s + 1 (read) and s + 3 (loaded); X unit of step s + 1 and
+  // the one being loaded
+  uint32_t wr = C::WSLOT, ww = C::AHEAD * C::WSLOT, xr = KU == 1 ? 0 : C::XUNIT,
+           xw = (KU == 1 ? 2 : C::AHEAD) * C::XUNIT;
+  auto next_w = [](uint32_t x) {
+    x += C::WSLOT;
+    return x == NS * C::WSLOT ? 0u : x;
+  };
+  auto next_x = [](uint32_t x) {
+    x += C::XUNIT;
+    return x == C::XU * C::XUNIT ? 0u : x;
+  };
+  // step s, H = s % 2
+  auto step = [&](auto full, auto half, int s, const P4Frag<XT, YT, KU>& f, P4Frag<XT, YT, KU>& nf) {
+    constexpr bool FULL = decltype(full)::value;
+    constexpr int H = decltype(half)::value, HX = KU == 1 ? H : 0;
+    if constexpr (FULL) p4_wait<(C::AHEAD - 2) * PER>();
+    else p4_wait_steps<PER, KU == 1 ? 0 : C::AHEAD - 2>(n_steps - 2 - s);
+    const lds_byte* nx[KU];
+    if constexpr (KU == 1) {
+      if (H == 1) xr = next_x(xr);  // step s + 1 starts a unit
+      nx[0] = rx0 + xr + px[1 - H];
+    } else {
+      nx[0] = rx0 + xr + px[0];
+      nx[KU - 1] = rx0 + xr + px[1];
+    }
+    // KU = 1: X unit s / 2 + 2 (its first k-block is step 2 (s / 2) + 4); KU = 2: unit s + 3
+    const bool load_w = FULL || s + C::AHEAD < n_steps;
+    const bool load_x = FULL || (KU == 1 ? s - H + 4 < n_steps : s + C::AHEAD < n_steps);
+    // the lane offsets pass through an empty asm statement, so that the addresses stay a scalar pointer
+    // plus a 32-bit offset (otherwise they become a pair of vector registers for every load)
+    uint32_t wl = wlane, xl[LX];
+    asm volatile("" : "+v"(wl));
+#pragma unroll
+    for (int r = 0; r < LX; ++r) {
+      xl[r] = xlane[HX][r];
+      asm volatile("" : "+v"(xl[r]));
+    }
+    p4_step<XT, YT, KU, LW, LX>(wp, xp[HX], wl, xl, load_w, load_x, dw0 + ww,
+                                dx0 + xw + HX * LX * 1024, rw0 + wr, nx, FULL || s + 1 < n_steps, f, nf, acc);
+#pragma unroll
+    for (int r = 0; r < LW; ++r) wp[r] += wstep;
+#pragma unroll
+    for (int r = 0; r < LX; ++r) xp[HX][r] += 128;
+    wr = next_w(wr);
+    ww = next_w(ww);
+    if (KU == 2) xr = next_x(xr);
+    if (KU == 2 || H == 1) xw = next_x(xw);
+  };
+  using yes_t = std::integral_constant<bool, true>;
+  using no_t = std::integral_constant<bool, false>;
+  using even_t = std::integral_constant<int, 0>;
+  using odd_t = std::integral_constant<int, 1>;
+  int s = 0;
+  for (; s + NS < n_steps; s += 2) {
+    step(yes_t{}, even_t{}, s, f0, f1);
+    step(yes_t{}, odd_t{}, s + 1, f1, f0);
+  }
+  for (; s < n_steps; s += 2) {  // the last steps
+    step(no_t{}, even_t{}, s, f0, f1);
+    if (s + 1 >= n_steps) break;
+    step(no_t{}, odd_t{}, s + 1, f1, f0);
+  }
+  p4_drain<XT, YT>(acc);
   __syncthreads();  // every wave is done with the slots: the staged tile and the scales reuse LDS
 
-  if constexpr (RS) {
-    rn_s[t] = a.row_scale[min(m0 + t, a.M - 1)];  // 256 threads, 256 rows
-    __syncthreads();
-  }
   {
     // the epilogue's thread indices pass through an empty asm statement, so that nothing computed
     // from them is hoisted above the k loop and kept live (spilled) across it
     int te = t;
     asm volatile("" : "+v"(te));
+    if constexpr (RS) {
+      if (te < C::BM) rn_s[te] = a.row_scale[min(m0 + te, a.M - 1)];
+      __syncthreads();
+    }
     const int je = te & 15, ge = (te >> 4) & 3, we = te >> 6, wne = we & 1, wme = we >> 1;
-    constexpr int COLS = EPI == EPI_SWIGLU ? 16 * XT : 32 * XT;  // staged columns
-    constexpr int NIT = COLS / 8;                                   // write-out items per thread
+    constexpr int NIT = C::COLS / 8;              // write-out items (16 bytes) per row
+    constexpr int NTH = (C::BM * NIT + 255) / 256;  // and per thread
     const int n_out = EPI == EPI_SWIGLU ? a.N / 2 : a.N;
     const int c0 = (EPI == EPI_SWIGLU ? nb0 * 8 : nb0 * 16);
     // The residual joins in the staging: lane (g, j)'s four columns of tile (x, y) are one 8-byte
@@ -344,7 +483,7 @@ __global__ __launch_bounds__(256, 1) void prefill_gemm4_kernel(GemmArgs a, int g
     [[maybe_unused]] uint2 rq[3][EPI == EPI_STORE ? XT : 1];
     auto load_res = [&](int y, uint2 (&dst)[EPI == EPI_STORE ? XT : 1]) {
       if constexpr (EPI == EPI_STORE) {
-        const int m = min(m0 + wme * 128 + y * 16 + je, a.M - 1);
+        const int m = min(m0 + (wme * YT + y) * 16 + je, a.M - 1);
 #pragma unroll
         for (int x = 0; x < XT; ++x) {
           const int n = min(c0 + (wne * XT + x) * 16 + 4 * ge, n_out - 4);
@@ -352,27 +491,30 @@ __global__ __launch_bounds__(256, 1) void prefill_gemm4_kernel(GemmArgs a, int g
         }
       }
     };
-    [[maybe_unused]] P4Rope<EPI == EPI_QKV ? XT : 1> rope;
+    [[maybe_unused]] P4Rope<C> rope;
     if constexpr (EPI == EPI_STORE) {
       if (res) {
         load_res(0, rq[0]);
-        load_res(1, rq[1]);
+        if (YT > 1) load_res(1, rq[1]);
       }
     } else if constexpr (EPI == EPI_QKV) {
-      p4_qkv_rope<XT>(a, nb0, m0, pos0, te, rope);
+      p4_qkv_rope<C>(a, nb0, m0, pos0, te, rope);
     }
     // stage: lane (g, j) of tile (x, y) holds output rows 16 (wn XT + x) + 4 g + e of token
-    // wm 128 + 16 y + j -- four consecutive columns (plain, q/k/v). For SwiGLU, rows r (gate) and
+    // 16 (wm YT + y) + j -- four consecutive columns (plain, q/k/v). For SwiGLU, rows r (gate) and
     // r + 8 (up) meet through a lane swap, after which lanes g and g + 2 hold the same four pairs:
     // lanes g < 2 finish pairs 0, 1 and lanes g >= 2 pairs 2, 3 of them (intermediate columns
     // 8 (wn XT + x) + 4 (g & 1) + 2 (g >> 1) + 0, 1).
 #pragma unroll
-    for (int y = 0; y < 8; ++y) {
-      const int mr = wme * 128 + y * 16 + je;
+    for (int y = 0; y < YT; ++y) {
+      // one row at a time: its accumulators are first read here
+#pragma unroll
+      for (int x = 0; x < XT; ++x) asm volatile("" : "+a"(acc[x][y])::"memory");
+      const int mr = (wme * YT + y) * 16 + je;
       const float sc = RS ? rn_s[mr] : 1.f;
       if constexpr (EPI == EPI_STORE) {
         __builtin_amdgcn_sched_barrier(0);  // keep each row's loads two rows ahead (not all hoisted)
-        if (res && y + 2 < 8) load_res(y + 2, rq[(y + 2) % 3]);
+        if (res && y + 2 < YT) load_res(y + 2, rq[(y + 2) % 3]);
       }
 #pragma unroll
       for (int x = 0; x < XT; ++x) {
@@ -392,7 +534,7 @@ __global__ __launch_bounds__(256, 1) void prefill_gemm4_kernel(GemmArgs a, int g
           const float u0 = hi ? up[2] : up[0], u1 = hi ? up[3] : up[1];
           const float o0 = rbf(pf_silu(rbf(g0))) * rbf(u0), o1 = rbf(pf_silu(rbf(g1))) * rbf(u1);
           const int col = (wne * XT + x) * 8 + 4 * (ge & 1) + 2 * (ge >> 1);
-          *(uint32_t*)(stage + mr * P4_ROW + col) = pack_bf16x2(o0, o1);
+          *(uint32_t*)(stage + mr * C::ROW + col) = pack_bf16x2(o0, o1);
         } else {
           if constexpr (EPI == EPI_STORE) {
             if (res) {
@@ -404,29 +546,29 @@ __global__ __launch_bounds__(256, 1) void prefill_gemm4_kernel(GemmArgs a, int g
             }
           }
           const int col = (wne * XT + x) * 16 + 4 * ge;
-          *(uint2*)(stage + mr * P4_ROW + col) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+          *(uint2*)(stage + mr * C::ROW + col) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
         }
       }
     }
     __syncthreads();
     if constexpr (EPI == EPI_QKV) {
-      p4_qkv_out<XT>(a, stage, nb0, m0, pos0, te, rope);
+      p4_qkv_out<C>(a, stage, nb0, m0, pos0, te, rope);
     } else {
       // write out: 8 columns (16 bytes) per item, a row's items on consecutive threads
       if (vec && n_out % 8 == 0) {  // uniform: every item is one whole 16-byte piece
-        for (int i = 0; i < NIT; ++i) {
+        for (int i = 0; i < NTH; ++i) {
           const int it = te + 256 * i, row = it / NIT, c8 = (it % NIT) * 8;
           const int m = m0 + row, n = c0 + c8;
-          if (m >= a.M || n >= n_out) continue;
-          *(uint4*)(a.Y + (size_t)m * a.ldy + n) = *(const uint4*)(stage + row * P4_ROW + c8);
+          if ((NTH * 256 != C::BM * NIT && it >= C::BM * NIT) || m >= a.M || n >= n_out) continue;
+          *(uint4*)(a.Y + (size_t)m * a.ldy + n) = *(const uint4*)(stage + row * C::ROW + c8);
         }
       } else {  // element by element (unaligned output or residual, or N not a multiple of 8)
-        for (int i = 0; i < NIT; ++i) {
+        for (int i = 0; i < NTH; ++i) {
           const int it = te + 256 * i, row = it / NIT, c8 = (it % NIT) * 8;
           const int m = m0 + row, n = c0 + c8;
-          if (m >= a.M || n >= n_out) continue;
+          if ((NTH * 256 != C::BM * NIT && it >= C::BM * NIT) || m >= a.M || n >= n_out) continue;
           Pack8 v;
-          v.u = *(const uint4*)(stage + row * P4_ROW + c8);
+          v.u = *(const uint4*)(stage + row * C::ROW + c8);
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
             if (n + e >= n_out) continue;
@@ -701,29 +843,72 @@ __global__ __launch_bounds__(256) void prefill_rowscale_kernel(const bf16_t* __r
   if (lane == 0) rn[row] = rsqrtf(acc / (float)K + eps);
 }
 
-static int launch_prefill_gemm4(GemmArgs a, int group, int pos0, int epi, int cus, hipStream_t s) {
-  const int xt = epi == EPI_QKV ? 6 : 8;  // weight tiles per wave: 192- or 256-column workgroup tiles
-  const int n_mt = (a.M + P4_BM - 1) / P4_BM;
-  const int n_nt = (a.N + 32 * xt - 1) / (32 * xt);
-  const int per_xcd = max((cus / 8) & ~3, 4);  // one workgroup per CU
-  const int sb_m = n_mt < 4 ? n_mt : 4;
-  const int sb_n = per_xcd / sb_m;
-  const int grid = 8 * sb_n * sb_m;
-#define PF4_LAUNCH(E, R, X)                                                                                     \
-  SSD_LAUNCH((prefill_gemm4_kernel<E, R, X>), dim3(grid), dim3(256), 0, s, a, group, n_mt, n_nt, pos0, sb_n, sb_m)
-#define PF4_SCALES(E, X)                   \
-  if (a.row_scale) PF4_LAUNCH(E, true, X); \
-  else PF4_LAUNCH(E, false, X);
-  if (epi == EPI_SWIGLU) {
-    PF4_SCALES(EPI_SWIGLU, 8);
-  } else if (epi == EPI_QKV) {
-    PF4_SCALES(EPI_QKV, 6);
-  } else {
-    PF4_SCALES(EPI_STORE, 8);
+// The tile shapes, largest first, and what a call with each costs: fixed + K / 64 * per-64-k cost *
+// tiles of the busiest CU (two tiles share a CU's time where two workgroups fit). The costs are a
+// least-squares fit (relative error) to the times of q/k/v, o, gate/up and down of the 1B, 8B and 70B shapes
+// at 23 M from 24 to 4096 with every shape (us, this card); the rule's choice is within 1.2 % of the
+// fastest shape on average there (worst 21 %). Large tiles move the fewest operand bytes per MFMA;
+// small ones put a short prompt's few rows on all CUs (M = 512, N = 4096, K = 14336: 32 tiles of 256
+// x 256 279 us, 256 of 128 x 64 90 us).
+struct PrefillTile {
+  int xt, yt, occ;
+  double fixed, one, two;  // us; per 64 k with one tile on a CU, with two side by side (occ 2)
+};
+constexpr PrefillTile PREFILL_TILES[] = {
+    {8, 8, 1, 14.2, 1.275, 0}, {6, 8, 1, 10.5, 1.032, 0},     {8, 4, 1, 3.0, 0.876, 0},
+    {6, 4, 1, 1.9, 0.746, 0},  {4, 4, 1, 4.0, 0.509, 0},      {4, 2, 1, 2.9, 0.364, 0},
+    {2, 2, 2, 2.7, 0.233, 0.418}, {1, 2, 2, 3.1, 0.178, 0.294}, {1, 1, 2, 4.2, 0.121, 0.208},
+};
+constexpr int N_PREFILL_TILES = sizeof(PREFILL_TILES) / sizeof(PREFILL_TILES[0]);
+
+static int pick_prefill_tile(int first, int M, int N, int K, int cus) {
+  int best = first;
+  double best_t = 0;
+  for (int i = first; i < N_PREFILL_TILES; ++i) {
+    const PrefillTile& p = PREFILL_TILES[i];
+    const int64_t tiles = ((int64_t)M + 32 * p.yt - 1) / (32 * p.yt) * (((int64_t)N + 32 * p.xt - 1) / (32 * p.xt));
+    const int64_t q = (tiles + cus - 1) / cus;  // tiles of the busiest CU
+    const double t = p.fixed + K / 64 * (p.occ == 2 ? q / 2 * p.two + q % 2 * p.one : q * p.one);
+    if (i == first || t < best_t) {
+      best = i;
+      best_t = t;
+    }
   }
-#undef PF4_SCALES
-#undef PF4_LAUNCH
+  return best;
+}
+
+template <int EPI, int XT, int YT, int KU, int NS, int OCC>
+static int launch_prefill_tile(const GemmArgs& a, int group, int pos0, int cus, hipStream_t s) {
+  const int n_mt = (a.M + 32 * YT - 1) / (32 * YT), n_nt = (a.N + 32 * XT - 1) / (32 * XT);
+  const int per_xcd = (n_mt * n_nt + 7) / 8, resident = max(cus / 8, 1) * OCC;
+  const int grid = 8 * min(per_xcd, resident);
+  const int band = min(n_mt, 4);
+  if (a.row_scale)
+    SSD_LAUNCH((prefill_gemm4_kernel<EPI, true, XT, YT, KU, NS, OCC>), dim3(grid), dim3(256), 0, s, a, group, n_mt, n_nt,
+               pos0, band);
+  else
+    SSD_LAUNCH((prefill_gemm4_kernel<EPI, false, XT, YT, KU, NS, OCC>), dim3(grid), dim3(256), 0, s, a, group, n_mt, n_nt,
+               pos0, band);
   return check_launch("prefill_gemm4");
+}
+
+// Ring depth: as many steps as fit LDS beside the other workgroup; short steps need the depth to cover
+// the memory latency (M = 100, N = 4096, K = 14336 on 32 x 64 tiles: 72 us with 4 slots, 44 with 6).
+template <int EPI>
+static int launch_prefill_gemm4(const GemmArgs& a, int group, int pos0, int cus, hipStream_t s) {
+  // (the largest tile's q/k/v write-out would spill registers across the k loop: not offered there)
+  switch (pick_prefill_tile(EPI == EPI_QKV ? 1 : 0, a.M, a.N, a.kb_total * 32, cus)) {
+    case 0:
+      if constexpr (EPI != EPI_QKV) return launch_prefill_tile<EPI, 8, 8, 1, 4, 1>(a, group, pos0, cus, s);
+    case 1: return launch_prefill_tile<EPI, 6, 8, 1, 4, 1>(a, group, pos0, cus, s);
+    case 2: return launch_prefill_tile<EPI, 8, 4, 1, 4, 1>(a, group, pos0, cus, s);
+    case 3: return launch_prefill_tile<EPI, 6, 4, 1, 4, 1>(a, group, pos0, cus, s);
+    case 4: return launch_prefill_tile<EPI, 4, 4, 2, 5, 1>(a, group, pos0, cus, s);
+    case 5: return launch_prefill_tile<EPI, 4, 2, 2, 6, 1>(a, group, pos0, cus, s);
+    case 6: return launch_prefill_tile<EPI, 2, 2, 2, 5, 2>(a, group, pos0, cus, s);
+    case 7: return launch_prefill_tile<EPI, 1, 2, 2, 6, 2>(a, group, pos0, cus, s);
+    default: return launch_prefill_tile<EPI, 1, 1, 2, 8, 2>(a, group, pos0, cus, s);
+  }
 }
 
 static int launch_prefill_gemm(GemmArgs a, int group, int pos0, int epi, hipStream_t s) {
@@ -735,7 +920,24 @@ static int launch_prefill_gemm(GemmArgs a, int group, int pos0, int epi, hipStre
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
     if (dev >= 0 && dev < 64) cus_of[dev] = cus;
   }
-  return launch_prefill_gemm4(a, group, pos0, epi, cus, s);
+  // the kernel's lane offsets into X are 32 bits over at most 8 rows: rows further apart than that go
+  // one by one
+  if (a.ldx >= (int64_t)1 << 27 && a.M > 1) {
+    for (int m = 0; m < a.M; ++m) {
+      GemmArgs r = a;
+      r.M = 1;
+      r.X += (size_t)m * a.ldx;
+      r.Y += (size_t)m * a.ldy;
+      if (a.residual) r.residual += (size_t)m * a.ldr;
+      if (a.row_scale) r.row_scale += m;
+      const int rc = launch_prefill_gemm(r, group, pos0 + m, epi, s);
+      if (rc) return rc;
+    }
+    return SSD_OK;
+  }
+  if (epi == EPI_SWIGLU) return launch_prefill_gemm4<EPI_SWIGLU>(a, group, pos0, cus, s);
+  if (epi == EPI_QKV) return launch_prefill_gemm4<EPI_QKV>(a, group, pos0, cus, s);
+  return launch_prefill_gemm4<EPI_STORE>(a, group, pos0, cus, s);
 }
 
 static int check_packed(int N, int K, int group) {
