@@ -36,7 +36,10 @@ from ssd.models.llama import MI355XLlama
 
 MAXD = 32        # ancestors per row (ssd_attn_max_depth)
 CHUNK = 64       # rows per kernel launch chain (GEMM column tiles of 16 x 4)
-PREFILL_MIN = 256     # causal prompt chunks at least this long run on the MFMA prefill kernels
+# Causal prompts at least this long run on the MFMA prefill kernels: everything past one decode forward of
+# CHUNK rows. One 8B layer, us: 64 rows 131 through the decode kernels, 117 through the prefill kernels; 100
+# rows 255 (two decode forwards) against 137; 32 rows 90 against 112.
+PREFILL_MIN = CHUNK + 1
 PREFILL_CHUNK = 4096  # prompt rows per ssd_prefill call
 
 
