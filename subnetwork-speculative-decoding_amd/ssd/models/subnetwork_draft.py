@@ -354,17 +354,19 @@ class SubnetworkDraftModel(nn.Module):
         return (self.layer_indices == list(range(s.layers)) and not self.bridge_specs and s.head_dim in (64, 128)
                 and s.hidden % 64 == 0 and s.inter % 64 == 0 and (s.heads * s.head_dim) % 64 == 0)
 
-    def prefill_chunk(self, ids: list, pos0: int, cache: KVCache, logits: bool) -> Optional[torch.Tensor]:
-        """ssd_prefill over prompt rows pos0 .. pos0 + len(ids) - 1 (at most PREFILL_CHUNK): K/V
-        of every layer into the cache, the final residual stream in the prefill workspace's h, and
-        with ``logits`` the last row's full-vocabulary logits ([1, V] view)."""
+    def prefill_chunk(self, ids, pos0: int, cache: KVCache, logits: bool) -> Optional[torch.Tensor]:
+        """ssd_prefill over prompt rows pos0 .. pos0 + len(ids) - 1 (at most PREFILL_CHUNK; ``ids`` a list
+        or a host int32 tensor): K/V of every layer into the cache, the final residual stream in the
+        prefill workspace's h, and with ``logits`` the last row's full-vocabulary logits ([1, V] view)."""
         m = len(ids)
         if m > PREFILL_CHUNK:
             raise ValueError(f"prefill chunk of {m} rows > {PREFILL_CHUNK}")
         pw = self._pw
         if pw is None or pw.m_cap < m:
             pw = self._pw = PrefillWorkspace(self.model, max(m, min(PREFILL_CHUNK, 1024)))
-        pw.ids[:m].copy_(torch.tensor(ids, dtype=torch.int32))
+        # from pinned memory, so that the layers are enqueued without waiting for the copy (the allocator
+        # keeps the block until the stream has read it)
+        pw.ids[:m].copy_(torch.as_tensor(ids, dtype=torch.int32).pin_memory(), non_blocking=True)
         _lib.call("ssd_prefill", self.model.native(cache.capacity), self.model.lm_head.data_ptr() if logits else None,
                   pw.native(cache), pw.ids.data_ptr(), m, int(pos0), ops.stream())
         return pw.logits if logits else None
@@ -514,31 +516,26 @@ class SubnetworkDraftModel(nn.Module):
             ids = ids[None]
         if ids.shape[0] != 1:
             raise ValueError("batch size 1 only (speculative decoding is batch 1)")
-        ids = ids[0].tolist()
-        q = len(ids)
+        q = ids.shape[1]
         cache = past_key_values
         if cache is None:
             cache = self.new_cache(q)
         cache.ensure(self.num_kv_heads, self.head_dim, self.model.device)
         past = cache.get_seq_length()
         cache.check_room(past + q)
-        pos = list(range(past, past + q)) if position_ids is None else torch.as_tensor(position_ids).reshape(-1).tolist()
+        pos = None if position_ids is None else torch.as_tensor(position_ids).reshape(-1).tolist()
+        if (tree_attention_mask is None and not output_bridge_states and q >= PREFILL_MIN and self.prefill_capable()
+                and (pos is None or pos == list(range(past, past + q)))):
+            return self._forward_prompt(ids[0], cache, logits_to_keep, compute_logits, past_key_values)
+        ids = ids[0].tolist()
+        if pos is None:
+            pos = list(range(past, past + q))
         prefix, anc = self.mask_to_rows(q, past, tree_attention_mask)
         ws = self.workspace(CHUNK)
         rows = Rows(CHUNK, self.model.device)
         hraw = torch.empty(q, self.d_model, dtype=torch.bfloat16, device=self.model.device)
         states: dict = {} if output_bridge_states else None
-        causal = tree_attention_mask is None and pos == list(range(past, past + q))
-        if causal and states is None and q >= PREFILL_MIN and self.prefill_capable():
-            # a long causal prompt: the MFMA prefill kernels, PREFILL_CHUNK rows per call
-            for c0 in range(0, q, PREFILL_CHUNK):
-                c1 = min(q, c0 + PREFILL_CHUNK)
-                self.prefill_chunk(ids[c0:c1], past + c0, cache, False)
-                hraw[c0:c1].copy_(self._pw.h[:c1 - c0])
-            q_done = q
-        else:
-            q_done = 0
-        for c0 in range(q_done, q, CHUNK):
+        for c0 in range(0, q, CHUNK):
             c1 = min(q, c0 + CHUNK)
             seen = [a for lst in anc[c0:c1] for a in lst] + [p - 1 for p in prefix[c0:c1]]
             if max(seen) >= past + c1:
@@ -559,18 +556,45 @@ class SubnetworkDraftModel(nn.Module):
         # hidden_states = the final-normed rows (reference :343); the decode path never needs
         # them (its head folds the norm), so they are computed here only
         hidden = torch.empty_like(hraw)
-        for c0 in range(0, q, CHUNK):
-            self.final_norm(hraw[c0:c0 + CHUNK], min(CHUNK, q - c0), hidden[c0:c0 + CHUNK])
+        if q:
+            self.final_norm(hraw, q, hidden)
         logits = None
         if compute_logits:
-            keep = hraw[-logits_to_keep:] if logits_to_keep > 0 else hraw
-            outs = []
-            for c0 in range(0, keep.shape[0], CHUNK):
-                part = keep[c0:c0 + CHUNK]
-                outs.append(self.head(part, part.shape[0], ws).clone())
-            logits = torch.cat(outs, 0)[None]
+            logits = self._head_rows(hraw[-logits_to_keep:] if logits_to_keep > 0 else hraw, ws)
         return DraftOutput(logits=logits, hidden_states=hidden[None], past_key_values=past_key_values,
                            bridge_states={k: v[None] for k, v in (states or {}).items()},
+                           vocab_ids=self.vocab_ids if compute_logits else None)
+
+    def _head_rows(self, h: torch.Tensor, ws: Workspace) -> torch.Tensor:
+        """The head over any number of rows of the final residual stream -> new bf16 logits [1, rows, V]."""
+        outs = [self.head(h[c0:c0 + CHUNK], min(CHUNK, h.shape[0] - c0), ws).clone()
+                for c0 in range(0, h.shape[0], CHUNK)]
+        return (outs[0] if len(outs) == 1 else torch.cat(outs, 0))[None]
+
+    def _forward_prompt(self, ids: torch.Tensor, cache: KVCache, logits_to_keep: int, compute_logits: bool,
+                        past_key_values: Optional[KVCache]) -> DraftOutput:
+        """forward() of a long causal prompt: the MFMA prefill kernels, PREFILL_CHUNK rows per call, one
+        final-norm launch per chunk, and the head on the rows asked for."""
+        q, past = ids.numel(), cache.get_seq_length()
+        ids = ids.cpu()
+        host = ids.to(torch.int32)
+        if ids.dtype == torch.int64 and not torch.equal(host.to(torch.int64), ids):
+            raise RuntimeError("token ids cannot be converted to int32 without overflow")
+        ws = self.workspace(CHUNK)
+        n_keep = 0 if not compute_logits else min(logits_to_keep, q) if logits_to_keep > 0 else q
+        hidden = torch.empty(q, self.d_model, dtype=torch.bfloat16, device=self.model.device)
+        keep = torch.empty(n_keep, self.d_model, dtype=torch.bfloat16, device=self.model.device)
+        for c0 in range(0, q, PREFILL_CHUNK):
+            c1 = min(q, c0 + PREFILL_CHUNK)
+            self.prefill_chunk(host[c0:c1], past + c0, cache, False)
+            self.final_norm(self._pw.h, c1 - c0, hidden[c0:c1])
+            k0 = max(c0, q - n_keep)
+            if k0 < c1:
+                keep[k0 - (q - n_keep):c1 - (q - n_keep)].copy_(self._pw.h[k0 - c0:c1 - c0])
+        logits = self._head_rows(keep, ws) if compute_logits else None
+        ws.check_faults()
+        cache.advance(q)
+        return DraftOutput(logits=logits, hidden_states=hidden[None], past_key_values=past_key_values, bridge_states={},
                            vocab_ids=self.vocab_ids if compute_logits else None)
 
     # ------------------------------------------------------------ persistence
