@@ -94,28 +94,107 @@ __device__ __forceinline__ uint32_t u4_get(const U4& r, int e) {
   return e == 0 ? r.x : e == 1 ? r.y : e == 2 ? r.z : r.w;
 }
 
-// ----------------------------------------------------------- block reductions (1024 threads)
-__device__ __forceinline__ float block_max(float v, float* sh) {
+// ----------------------------------------------------------- reductions
+// Workgroup reductions put the 16 waves' partials into `sh` and pass one barrier; `sh` belongs to that
+// one reduction, so that none of them needs a second barrier before it is used again.
+//
+// Inside a wave, values move between lanes by DPP and the permlane swaps (VALU) rather than by shuffles,
+// which all go through LDS: with 32 waves on a CU the ~60 exchanges of an acceptance pass cost more there
+// than its loads. Steps 1, 2, 4, 8 pair lanes by quad permutation and the mirrors of 8 and 16 lanes (the
+// lanes of each half hold one value by then, so a mirror reaches the same partner value as an xor),
+// steps 16 and 32 by the swaps: every lane ends with the same value, and a sum adds the same pairs in
+// the same order as a butterfly of xor shuffles.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+}
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140;
+
+template <typename T>
+struct Words {
+  static constexpr int N = sizeof(T) / 4;
+  uint32_t w[N];
+};
+
+// r0 and r1 of each lane: its own value and its partner's at the given step (in either order).
+template <int STEP, typename T>
+__device__ __forceinline__ void wave_pair(T v, T& r0, T& r1) {
+  const Words<T> x = __builtin_bit_cast(Words<T>, v);
+  Words<T> a, b;
 #pragma unroll
-  for (int o = 32; o; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
+  for (int i = 0; i < Words<T>::N; ++i) {
+    a.w[i] = x.w[i];
+    if constexpr (STEP == 1) b.w[i] = dpp<DPP_XOR1>(x.w[i]);
+    else if constexpr (STEP == 2) b.w[i] = dpp<DPP_XOR2>(x.w[i]);
+    else if constexpr (STEP == 4) b.w[i] = dpp<DPP_HALF_MIRROR>(x.w[i]);
+    else if constexpr (STEP == 8) b.w[i] = dpp<DPP_MIRROR>(x.w[i]);
+    else {
+      const auto p = STEP == 16 ? __builtin_amdgcn_permlane16_swap(x.w[i], x.w[i], false, false)
+                                : __builtin_amdgcn_permlane32_swap(x.w[i], x.w[i], false, false);
+      a.w[i] = p[0];
+      b.w[i] = p[1];
+    }
+  }
+  r0 = __builtin_bit_cast(T, a);
+  r1 = __builtin_bit_cast(T, b);
+}
+
+// All 64 lanes reduced by a commutative `op`.
+template <typename T, class Op>
+__device__ __forceinline__ T wave_reduce(T v, Op op) {
+  T a, b;
+  wave_pair<1>(v, a, b);
+  wave_pair<2>(op(a, b), a, b);
+  wave_pair<4>(op(a, b), a, b);
+  wave_pair<8>(op(a, b), a, b);
+  wave_pair<16>(op(a, b), a, b);
+  wave_pair<32>(op(a, b), a, b);
+  return op(a, b);
+}
+
+__device__ __forceinline__ float wave_max(float v) {
+  return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
+}
+
+template <typename T>
+__device__ __forceinline__ T wave_sum(T v) {
+  return wave_reduce(v, [](T a, T b) { return a + b; });
+}
+
+// Inclusive prefix sum over the lanes: DPP shifts inside each row of 16, then the rows' last lanes
+// broadcast to the rows above (CTRL 0x142 / 0x143: lane 15 of each row, lane 31).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint64_t dpp64(uint64_t v) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWS, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, ROWS, 0xf, false);
+  return (uint64_t)hi << 32 | lo;
+}
+__device__ __forceinline__ uint64_t wave_scan(uint64_t v) {
+  v += dpp64<0x111, 0xf>(v);
+  v += dpp64<0x112, 0xf>(v);
+  v += dpp64<0x114, 0xf>(v);
+  v += dpp64<0x118, 0xf>(v);
+  v += dpp64<0x142, 0xa>(v);
+  v += dpp64<0x143, 0xc>(v);
+  return v;
+}
+
+__device__ __forceinline__ float block_max(float v, float* sh) {
+  v = wave_max(v);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
   float r = sh[0];
+#pragma unroll
   for (int i = 1; i < 16; ++i) r = fmaxf(r, sh[i]);
-  __syncthreads();
   return r;
 }
 
-// Fixed-order sums: butterfly inside each wave, then the 16 wave sums in order.
+// The waves' sums in order, once they are all in `sh`.
 template <typename T>
-__device__ __forceinline__ T block_sum(T v, T* sh) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) v += __shfl_xor(v, o);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-  __syncthreads();
+__device__ __forceinline__ T sum16(const T* sh) {
   T r = sh[0];
+#pragma unroll
   for (int i = 1; i < 16; ++i) r += sh[i];
-  __syncthreads();
   return r;
 }
 
@@ -130,24 +209,32 @@ __device__ __forceinline__ bool better(float ka, int ia, float kb, int ib) {
 
 constexpr int NO_IDX = 0x7fffffff;
 
-// Largest key, lowest index among equal keys. Every thread gets the result.
-__device__ __forceinline__ KeyIdx block_argmax(float key, int idx, KeyIdx* sh) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const float k2 = __shfl_xor(key, o);
-    const int i2 = __shfl_xor(idx, o);
-    if (better(k2, i2, key, idx)) {
-      key = k2;
-      idx = i2;
+// Largest key, lowest index among equal keys (a strict order, so any order of merging gives the same).
+__device__ __forceinline__ KeyIdx wave_argmax(float k, int i) {
+  return wave_reduce(KeyIdx{k, i}, [](KeyIdx a, KeyIdx b) { return better(a.key, a.idx, b.key, b.idx) ? a : b; });
+}
+
+// f(e) for every set bit e of the lanes' 4-bit masks, all lanes taking their next one together. The
+// columns of a nucleus are few (2 % of 128256 at T 0.7 and top_p 0.9), so a wave that looked at its lanes'
+// four columns one after another would run the logarithms of a draw four times, mostly for a lane or two.
+template <class F>
+__device__ __forceinline__ void for_active(uint32_t mask, F f) {
+  while (__ballot(mask != 0)) {
+    if (mask) {
+      f(__ffs((int)mask) - 1);
+      mask &= mask - 1;
     }
   }
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = KeyIdx{key, idx};
-  __syncthreads();
-  KeyIdx r = sh[0];
-  for (int i = 1; i < 16; ++i)
-    if (better(sh[i].key, sh[i].idx, r.key, r.idx)) r = sh[i];
-  __syncthreads();
-  return r;
+}
+__device__ __forceinline__ float get4(const float (&v)[4], int e) {
+  return e == 0 ? v[0] : e == 1 ? v[1] : e == 2 ? v[2] : v[3];
+}
+
+// The best of the 16 waves' records in `sh`, by one wave.
+__device__ __forceinline__ KeyIdx argmax16(const KeyIdx* sh) {
+  const int lane = threadIdx.x & 63;
+  const KeyIdx v = lane < 16 ? sh[lane] : KeyIdx{-1.f, NO_IDX};
+  return wave_argmax(v.key, v.idx);
 }
 
 // Inclusive prefix sum over the 1024 threads (thread order).
@@ -166,24 +253,15 @@ __device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* sh) {
   return v + add;
 }
 
-__device__ __forceinline__ uint64_t block_scan64(uint64_t v, uint64_t* sh) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint64_t n = __shfl_up(v, o);
-    if (lane >= o) v += n;
-  }
-  if (lane == 63) sh[w] = v;
-  __syncthreads();
-  uint64_t add = 0;
-  for (int i = 0; i < w; ++i) add += sh[i];
-  __syncthreads();
-  return v + add;
-}
-
 // ------------------------------------------------------------------------ workspace
 // One caller-provided buffer, carved per (rows, chunks). Histograms are cleared by the first
 // launch of each warp; every other array is fully written before it is read.
+struct NodeKids {  // children of a verify node that the acceptance considers, in rank order
+  int n;
+  int kid[SMP_MAXK];
+  int tok[SMP_MAXK];
+};
+
 struct SmpWs {
   float2* stats;      // [rows][C] chunk (max, sum exp) of logits / T
   uint64_t* coarse;   // [rows][256] mass by key high byte
@@ -196,6 +274,7 @@ struct SmpWs {
   KeyIdx* bon;        // [rows][SMP_MAXK + 1][C] bonus draw partials per rejection state
   double* s0;         // [rows][C] mass of q0 per chunk
   int* supp;          // [rows][C] support of q0 per chunk
+  NodeKids* kids;     // [rows] each verify row's children, written by the first acceptance pass
   int C;
 };
 
@@ -221,6 +300,7 @@ static int64_t smp_layout(int rows, int C, char* base, SmpWs* ws) {
   w.bon = (KeyIdx*)take(R * (SMP_MAXK + 1) * CC * sizeof(KeyIdx));
   w.s0 = (double*)take(R * CC * 8);
   w.supp = (int*)take(R * CC * 4);
+  w.kids = (NodeKids*)take(R * (int64_t)sizeof(NodeKids));
   w.C = C;
   if (ws) *ws = w;
   return off;
@@ -268,8 +348,10 @@ __device__ __forceinline__ uint32_t key_bf(uint32_t k) { return k ^ ((k & 0x8000
 
 // The probability of a logit and its fixed-point mass: one code path for every use, so a
 // value and the mass accumulated for it always agree bit for bit.
+__device__ __forceinline__ float scaled_of(uint32_t h, float temp) { return bf2f((bf16_t)h) / temp; }
+__device__ __forceinline__ float prob_scaled(float x, float M, float S) { return expf(x - M) / S; }
 __device__ __forceinline__ float prob_of(uint32_t h, float temp, float M, float S) {
-  return expf(bf2f((bf16_t)h) / temp - M) / S;
+  return prob_scaled(scaled_of(h, temp), M, S);
 }
 __device__ __forceinline__ uint64_t mass_of(float p) { return __double2ull_rn((double)p * 0x1p52); }
 
@@ -286,48 +368,76 @@ __device__ __forceinline__ void load4_bf16(const bf16_t* row, int i, int n, uint
   }
 }
 
-struct WarpShared {
-  float red_f[16];
-  uint32_t red_u[16];
-  uint64_t red_l[16];
-  uint64_t histm[256];
-  uint32_t histc[256];
-  float M, S;
-  int cut;
+// Row max and sum exp from the chunk partials, by one wave (C <= 256). The sum's order is that of a
+// 1024-thread workgroup over the chunk index: a butterfly per 64 chunks, then those in order.
+__device__ __forceinline__ void row_stats(const float2* st, int C, float& M, float& S) {
+  const int lane = threadIdx.x & 63;
+  float2 v[SMP_MAXC / 64];
+  float m = -INFINITY;
+#pragma unroll
+  for (int u = 0; u < SMP_MAXC / 64; ++u) {
+    v[u] = make_float2(-INFINITY, 0.f);
+    if (64 * u < C && lane + 64 * u < C) v[u] = st[lane + 64 * u];
+    m = fmaxf(m, v[u].x);
+  }
+  M = wave_max(m);
+  S = 0.f;
+#pragma unroll
+  for (int u = 0; u < SMP_MAXC / 64; ++u)
+    if (u == 0 || 64 * u < C) {
+      const float e = wave_sum(lane + 64 * u < C && v[u].x != -INFINITY ? v[u].y * expf(v[u].x - M) : 0.f);
+      S = u == 0 ? e : S + e;
+    }
+}
+
+// Scan of a 256-bin histogram from the largest key down, by one wave: lane l holds the masses of bins
+// 255 - 4 l - e. cut: the bin with the first entry whose preceding mass exceeds T (-1 when the whole
+// histogram fits under T); above: the mass of the bins over it, plus `base`; total: base plus all.
+struct Cut {
+  int bin;
   uint64_t above, total;
 };
 
-// Row max and sum exp from the chunk partials (fixed order: block reduction over chunk index).
-__device__ __forceinline__ void row_stats(const float2* st, int C, WarpShared& sh, float& M, float& S) {
-  const int t = threadIdx.x;
-  const float2 v = t < C ? st[t] : make_float2(-INFINITY, 0.f);
-  M = block_max(v.x, sh.red_f);
-  S = block_sum<float>(t < C && v.x != -INFINITY ? v.y * expf(v.x - M) : 0.f, sh.red_f);
+__device__ __forceinline__ Cut wave_cut(const uint64_t (&v)[4], uint64_t base, uint64_t T) {
+  const int lane = threadIdx.x & 63;
+  const uint64_t sum = v[0] + v[1] + v[2] + v[3];
+  const uint64_t incl = wave_scan(sum);
+  Cut r{-1, 0, base + __shfl(incl, 63)};
+  uint64_t before = base + incl - sum;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (v[e] > 0 && before <= T && T < before + v[e]) {
+      r.bin = 255 - 4 * lane - e;
+      r.above = before;
+    }
+    before += v[e];
+  }
+  const uint64_t found = __ballot(r.bin >= 0);
+  if (found) {
+    const int src = __ffsll((unsigned long long)found) - 1;
+    r.bin = __shfl(r.bin, src);
+    r.above = __shfl(r.above, src);
+  }
+  return r;
 }
 
-// Scan a 256-bin histogram (bin masses from mass_fn(bin)) from the largest key down: the bin
-// holding the first entry whose preceding mass exceeds T. Sets sh.cut (-1 when the whole
-// histogram fits under T), sh.above (mass of the bins above the cut bin, plus `base`) and
-// sh.total.
-template <typename MassFn>
-__device__ __forceinline__ void cut_scan(MassFn mass_fn, uint64_t base, uint64_t T, WarpShared& sh) {
-  const int t = threadIdx.x;
-  const int b = 255 - t;
-  const uint64_t v = t < 256 ? mass_fn(b) : 0ull;
-  const uint64_t incl = block_scan64(v, sh.red_l);
-  if (t == 0) sh.cut = -1;
-  if (t == 255) sh.total = base + incl;
-  __syncthreads();
-  if (t < 256 && v > 0 && base + incl - v <= T && T < base + incl) {
-    sh.cut = b;
-    sh.above = base + incl - v;
-  }
-  __syncthreads();
+// This lane's four bins of a histogram, in wave_cut's order.
+template <typename T>
+__device__ __forceinline__ void load_bins(const T* hist, T (&v)[4]) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = hist[255 - 4 * (threadIdx.x & 63) - e];
 }
+
+// The four launches of a warp are chains of memory round trips and reductions rather than bytes (16 rows
+// of 128256: 11 MB). What concerns the whole row -- its statistics, the cut -- is therefore done by the
+// first wave of each workgroup while the others load their logits, with one barrier behind it; scanning
+// the histograms with all 1024 threads took two barriers and a serial pass over the 16 waves each
+// (us for 16 rows, before / after: stats 5.6 / 4.9, coarse 8.2 / 6.2, fine 5.4 / 3.9, final
+// 16.3 / 10.0).
 
 // L0: chunk max / sum exp; the first chunk of each row clears the row's histograms.
 __global__ __launch_bounds__(SMP_THREADS) void warp_stats_kernel(WarpArgs a) {
-  __shared__ WarpShared sh;
+  __shared__ float red_m[16], red_s[16];
   int F, base;
   frontier_rows(a.meta, a.level, a.rows, F, base);
   const int f = blockIdx.y, c = blockIdx.x, t = threadIdx.x;
@@ -342,66 +452,87 @@ __global__ __launch_bounds__(SMP_THREADS) void warp_stats_kernel(WarpArgs a) {
   float x[4], m = -INFINITY;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    x[e] = i + e < a.n ? bf2f((bf16_t)h[e]) / a.temp : -INFINITY;
+    x[e] = i + e < a.n ? scaled_of(h[e], a.temp) : -INFINITY;
     m = fmaxf(m, x[e]);
   }
-  const float M = block_max(m, sh.red_f);
+  const float M = block_max(m, red_m);
   float s = 0.f;
 #pragma unroll
   for (int e = 0; e < 4; ++e) s += i + e < a.n ? expf(x[e] - M) : 0.f;
-  const float S = block_sum<float>(s, sh.red_f);
-  if (t == 0) a.ws.stats[(size_t)f * a.ws.C + c] = make_float2(M, S);
+  s = wave_sum(s);
+  if ((t & 63) == 0) red_s[t >> 6] = s;
+  __syncthreads();
+  if (t == 0) a.ws.stats[(size_t)f * a.ws.C + c] = make_float2(M, sum16(red_s));
 }
 
-// L1: mass / count histogram of the key high byte.
+// L1: mass histogram of the key high byte. A row's logits fall into few of the 256 bins (sign and
+// exponent), so each bin has HCOPY counters side by side, picked by the thread.
+constexpr int HCOPY = 8;
 __global__ __launch_bounds__(SMP_THREADS) void warp_coarse_kernel(WarpArgs a) {
-  __shared__ WarpShared sh;
+  __shared__ uint64_t hist[256 * HCOPY];
+  __shared__ float M_sh, S_sh;
   int F, base;
   frontier_rows(a.meta, a.level, a.rows, F, base);
   const int f = blockIdx.y, c = blockIdx.x, t = threadIdx.x;
   if (f >= F) return;
-  float M, S;
-  row_stats(a.ws.stats + (size_t)f * a.ws.C, a.ws.C, sh, M, S);
-  if (t < 256) sh.histm[t] = 0;
-  __syncthreads();
   const int i = c * SMP_CHUNK + t * 4;
   uint32_t h[4];
   load4_bf16(a.logits + (size_t)f * a.ld, i, a.n, h);
+  if (t < 64) {
+    float M, S;
+    row_stats(a.ws.stats + (size_t)f * a.ws.C, a.ws.C, M, S);
+    if (t == 0) {
+      M_sh = M;
+      S_sh = S;
+    }
+  }
+  for (int b = t; b < 256 * HCOPY; b += SMP_THREADS) hist[b] = 0;
+  __syncthreads();
+  const float M = M_sh, S = S_sh;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     if (i + e >= a.n) continue;
-    const uint32_t bin = bf_key(h[e]) >> 8;
-    atomicAdd((unsigned long long*)&sh.histm[bin], (unsigned long long)mass_of(prob_of(h[e], a.temp, M, S)));
+    const uint64_t w = mass_of(prob_of(h[e], a.temp, M, S));
+    if (w) atomicAdd((unsigned long long*)&hist[(bf_key(h[e]) >> 8) * HCOPY + t % HCOPY], (unsigned long long)w);
   }
   __syncthreads();
-  if (t < 256 && sh.histm[t])
-    atomicAdd((unsigned long long*)&a.ws.coarse[(size_t)f * 256 + t], (unsigned long long)sh.histm[t]);
+  if (t < 256) {
+    uint64_t w = 0;
+#pragma unroll
+    for (int u = 0; u < HCOPY; ++u) w += hist[t * HCOPY + u];
+    if (w) atomicAdd((unsigned long long*)&a.ws.coarse[(size_t)f * 256 + t], (unsigned long long)w);
+  }
 }
 
 // L2: inside the coarse cut bin, count histogram of the key low byte (row total and per chunk).
 __global__ __launch_bounds__(SMP_THREADS) void warp_fine_kernel(WarpArgs a) {
-  __shared__ WarpShared sh;
+  __shared__ uint32_t hist[256];
+  __shared__ int cut_sh;
   int F, base;
   frontier_rows(a.meta, a.level, a.rows, F, base);
   const int f = blockIdx.y, c = blockIdx.x, t = threadIdx.x;
   if (f >= F) return;
-  const uint64_t* coarse = a.ws.coarse + (size_t)f * 256;
-  cut_scan([&](int b) { return coarse[b]; }, 0ull, a.T, sh);
-  const int cut = sh.cut;
-  if (cut < 0) return;  // everything fits under top_p (uniform per block)
-  if (t < 256) sh.histc[t] = 0;
-  __syncthreads();
   const int i = c * SMP_CHUNK + t * 4;
   uint32_t h[4];
   load4_bf16(a.logits + (size_t)f * a.ld, i, a.n, h);
+  if (t < 64) {
+    uint64_t v[4];
+    load_bins(a.ws.coarse + (size_t)f * 256, v);
+    const Cut cut = wave_cut(v, 0ull, a.T);
+    if (t == 0) cut_sh = cut.bin;
+  }
+  if (t < 256) hist[t] = 0;
+  __syncthreads();
+  const int cut = cut_sh;
+  if (cut < 0) return;  // everything fits under top_p (uniform per block)
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const uint32_t k = bf_key(h[e]);
-    if (i + e < a.n && (int)(k >> 8) == cut) atomicAdd(&sh.histc[k & 255], 1u);
+    if (i + e < a.n && (int)(k >> 8) == cut) atomicAdd(&hist[k & 255], 1u);
   }
   __syncthreads();
   if (t < 256) {
-    const uint32_t v = sh.histc[t];
+    const uint32_t v = hist[t];
     a.ws.finec[((size_t)f * a.ws.C + c) * 256 + t] = v;
     if (v) atomicAdd(&a.ws.fine[(size_t)f * 256 + t], v);
   }
@@ -409,12 +540,11 @@ __global__ __launch_bounds__(SMP_THREADS) void warp_fine_kernel(WarpArgs a) {
 
 // L3: probabilities out (renormalised survivors when top_p < 1); zeros outside a subset.
 __global__ __launch_bounds__(SMP_THREADS) void warp_final_kernel(WarpArgs a) {
-  __shared__ WarpShared sh;
-  __shared__ uint32_t cut_key_sh, c_keep_sh, prefix_sh;
-  __shared__ uint64_t kept_sh;
+  __shared__ float M_sh, S_sh, scale_sh;
+  __shared__ uint32_t cut_key_sh, c_keep_sh, prefix_sh, ties_sh[16];
   int F, base;
   frontier_rows(a.meta, a.level, a.rows, F, base);
-  const int f = blockIdx.y, c = blockIdx.x, t = threadIdx.x;
+  const int f = blockIdx.y, c = blockIdx.x, t = threadIdx.x, lane = t & 63;
   if (f >= F) return;
   float* out = a.out + (size_t)(base + f) * a.ldo;
   if (a.vocab) {  // tokens outside the subset have probability 0
@@ -424,68 +554,89 @@ __global__ __launch_bounds__(SMP_THREADS) void warp_final_kernel(WarpArgs a) {
       if (y0 + e < a.V && a.inv[y0 + e] < 0) out[y0 + e] = 0.f;
   }
   if (c * SMP_CHUNK >= a.n) return;  // a zero-fill-only chunk (uniform per block)
-  float M, S;
-  row_stats(a.ws.stats + (size_t)f * a.ws.C, a.ws.C, sh, M, S);
-  uint32_t cut_key = 0, c_keep = 0xffffffffu, prefix = 0;
-  float scale = 1.f;
-  if (a.top_p < 1.f) {
-    const uint64_t* coarse = a.ws.coarse + (size_t)f * 256;
-    cut_scan([&](int b) { return coarse[b]; }, 0ull, a.T, sh);
-    if (sh.cut < 0) {  // keep all: renormalise by the total mass
-      scale = (float)(1.0 / ((double)sh.total * 0x1p-52));
-    } else {
-      const int cb = sh.cut;
-      const uint64_t above = sh.above;
-      const uint32_t* fine = a.ws.fine + (size_t)f * 256;
-      // mass of fine bin b = count * mass of that exact logit
-      cut_scan([&](int b) {
-        const uint32_t n = fine[b];
-        return n ? (uint64_t)n * mass_of(prob_of(key_bf(((uint32_t)cb << 8) | (uint32_t)b), a.temp, M, S)) : 0ull;
-      }, above, a.T, sh);
-      if (t == 0) {
-        const int fb = sh.cut < 0 ? 0 : sh.cut;  // always found: the coarse bin's mass straddles T
-        const uint32_t key = ((uint32_t)cb << 8) | (uint32_t)fb;
-        const uint32_t n_t = fine[fb];
-        const uint64_t w = mass_of(prob_of(key_bf(key), a.temp, M, S));
-        const uint64_t C3 = sh.cut < 0 ? above : sh.above;
-        uint64_t keep = n_t;
-        if (w > 0 && a.T >= C3) keep = min((uint64_t)n_t, (a.T - C3) / w + 1ull);
-        cut_key_sh = key;
-        c_keep_sh = (uint32_t)keep;
-        kept_sh = C3 + keep * w;
-      }
-      __syncthreads();
-      cut_key = cut_key_sh;
-      c_keep = c_keep_sh;
-      scale = (float)(1.0 / ((double)kept_sh * 0x1p-52));
-      // ties of the cut key in earlier chunks
-      const uint32_t fb = cut_key & 255;
-      const uint32_t v = t < c ? a.ws.finec[((size_t)f * a.ws.C + t) * 256 + fb] : 0u;
-      const uint32_t pre = block_sum<uint32_t>(v, (uint32_t*)sh.red_u);
-      if (t == 0) prefix_sh = pre;
-      __syncthreads();
-      prefix = prefix_sh;
-    }
-  }
   const int i = c * SMP_CHUNK + t * 4;
   uint32_t h[4];
   load4_bf16(a.logits + (size_t)f * a.ld, i, a.n, h);
-  // column rank of this thread's ties of the cut key
-  uint32_t ties = 0;
+  if (t < 64) {  // the row's statistics and cut
+    float M, S, scale = 1.f;
+    uint64_t cm[4];
+    uint32_t fn[4];
+    if (a.top_p < 1.f) {  // loaded beside the statistics; the fine histogram is all zeros without a cut
+      load_bins(a.ws.coarse + (size_t)f * 256, cm);
+      load_bins(a.ws.fine + (size_t)f * 256, fn);
+    }
+    row_stats(a.ws.stats + (size_t)f * a.ws.C, a.ws.C, M, S);
+    uint32_t key = 0, c_keep = 0xffffffffu, prefix = 0;
+    if (a.top_p < 1.f) {
+      const Cut cc = wave_cut(cm, 0ull, a.T);
+      if (cc.bin < 0) {  // keep all: renormalise by the total mass
+        scale = (float)(1.0 / ((double)cc.total * 0x1p-52));
+      } else {
+        const uint32_t* fine = a.ws.fine + (size_t)f * 256;
+        // mass of fine bin b = count * mass of that exact logit
+        uint64_t v[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) ties += (i + e < a.n && bf_key(h[e]) == cut_key) ? 1u : 0u;
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t b = 255 - 4 * lane - e, n = fn[e];
+          v[e] = n ? (uint64_t)n * mass_of(prob_of(key_bf(((uint32_t)cc.bin << 8) | b), a.temp, M, S)) : 0ull;
+        }
+        const Cut fc = wave_cut(v, cc.above, a.T);
+        const int fb = fc.bin < 0 ? 0 : fc.bin;  // always found: the coarse bin's mass straddles T
+        key = ((uint32_t)cc.bin << 8) | (uint32_t)fb;
+        // ties of the cut key in earlier chunks
+        uint32_t n_before = 0;
+        for (int u = lane; u < c; u += 64) n_before += a.ws.finec[((size_t)f * a.ws.C + u) * 256 + fb];
+        const uint32_t n_t = fine[fb];
+        const uint64_t w = mass_of(prob_of(key_bf(key), a.temp, M, S));
+        const uint64_t C3 = fc.bin < 0 ? cc.above : fc.above;
+        uint64_t keep = n_t;
+        if (w > 0 && a.T >= C3) keep = min((uint64_t)n_t, (a.T - C3) / w + 1ull);
+        c_keep = (uint32_t)keep;
+        scale = (float)(1.0 / ((double)(C3 + keep * w) * 0x1p-52));
+        prefix = wave_sum(n_before);
+      }
+    }
+    if (t == 0) {
+      M_sh = M;
+      S_sh = S;
+      scale_sh = scale;
+      cut_key_sh = key;
+      c_keep_sh = c_keep;
+      prefix_sh = prefix;
+    }
+  }
+  float x[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = scaled_of(h[e], a.temp);
+  __syncthreads();
+  const float M = M_sh, S = S_sh, scale = scale_sh;
+  const uint32_t cut_key = cut_key_sh, c_keep = c_keep_sh;
+  // column rank of this thread's ties of the cut key (columns ascend with the thread, then e)
   uint32_t rank = 0;
-  if (a.top_p < 1.f && c_keep != 0xffffffffu) rank = prefix + block_scan(ties, sh.red_u) - ties;
+  const bool cut = a.top_p < 1.f && c_keep != 0xffffffffu;  // uniform per block
+  if (cut) {
+    uint32_t in_wave = 0, before = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint64_t m = __ballot(i + e < a.n && bf_key(h[e]) == cut_key);
+      in_wave += __popcll(m);
+      before += __popcll(m & ((1ull << lane) - 1));
+    }
+    if (lane == 0) ties_sh[t >> 6] = in_wave;
+    __syncthreads();
+    rank = prefix_sh + before;
+    for (int w = 0; w < t >> 6; ++w) rank += ties_sh[w];
+  }
   float p[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const uint32_t k = bf_key(h[e]);
     bool keep = true;
-    if (a.top_p < 1.f && c_keep != 0xffffffffu) {
+    if (cut) {
       keep = k > cut_key;
       if (k == cut_key && i + e < a.n) keep = rank++ < c_keep;
     }
-    const float pv = prob_of(h[e], a.temp, M, S);
+    const float pv = prob_scaled(x[e], M, S);
     p[e] = keep ? (a.top_p < 1.f ? pv * scale : pv) : 0.f;
   }
   if (!a.vocab && i + 3 < a.n) {
@@ -523,15 +674,38 @@ __device__ __forceinline__ void load4_f32(const float* row, int i, int n, float 
   }
 }
 
+// The k best of the records each lane holds 4 of, best first: out[r] from lane 0.
+__device__ __forceinline__ void wave_topk(float (&kk)[4], int (&ki)[4], int k, KeyIdx* out) {
+  for (int r = 0; r < k; ++r) {
+    float bk = kk[0];
+    int bi = ki[0];
+#pragma unroll
+    for (int e = 1; e < 4; ++e)
+      if (better(kk[e], ki[e], bk, bi)) {
+        bk = kk[e];
+        bi = ki[e];
+      }
+    const KeyIdx w = wave_argmax(bk, bi);
+    if ((threadIdx.x & 63) == 0) out[r] = w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (ki[e] == w.idx) {
+        kk[e] = -1.f;
+        ki[e] = NO_IDX;
+      }
+  }
+}
+
 // Per chunk: the k largest keys q(y) / E(y) (E ~ Exp(1) from the PROPOSE stream) and the
-// support size. Keys of one thread are its 4 columns; the chunk's top k are popped one at a
-// time by block argmax.
+// support size. Every wave takes the k best of its 256 columns, then the first wave the k best of the
+// 16 lists: one barrier however large k is (a workgroup-wide maximum per draw took two each: 9.4 us for
+// 6 rows of 128256 and k = 2, now 7.0).
 __global__ __launch_bounds__(SMP_THREADS) void gumbel_chunk_kernel(TopkArgs a) {
-  __shared__ KeyIdx red[16];
+  __shared__ KeyIdx list[16][SMP_MAXK];
   __shared__ int red_i[16];
   int F, base;
   frontier_rows(a.meta, a.level, a.rows, F, base);
-  const int f = blockIdx.y, c = blockIdx.x, t = threadIdx.x;
+  const int f = blockIdx.y, c = blockIdx.x, t = threadIdx.x, lane = t & 63;
   if (f >= F) return;
   const float* q = a.q + (size_t)(base + f) * a.ldq;
   const int i = c * SMP_CHUNK + t * 4;
@@ -540,99 +714,83 @@ __global__ __launch_bounds__(SMP_THREADS) void gumbel_chunk_kernel(TopkArgs a) {
   const U4 r = rng_block(a.rng, (uint32_t)(i >> 2), (uint32_t)f | ((uint32_t)a.level << 16), TAG_PROPOSE);
   float kk[4];
   int ki[4];
-  int supp = 0;
+  uint32_t on = 0;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const bool on = i + e < a.V && v[e] > 0.f;
-    supp += on;
-    kk[e] = on ? v[e] / exp1_from_bits(u4_get(r, e)) : -1.f;
-    ki[e] = on ? i + e : NO_IDX;
+    on |= (uint32_t)(i + e < a.V && v[e] > 0.f) << e;
+    kk[e] = -1.f;
+    ki[e] = NO_IDX;
   }
-  const int support = block_sum<int>(supp, red_i);
-  KeyIdx* cand = a.ws.cand + ((size_t)f * a.ws.C + c) * SMP_MAXK;
-  for (int j = 0; j < a.k; ++j) {
-    // this thread's best remaining column
-    int b = 0;
+  int supp = __popc(on);
+  for_active(on, [&](int e) {
+    const float key = get4(v, e) / exp1_from_bits(u4_get(r, e));
 #pragma unroll
-    for (int e = 1; e < 4; ++e)
-      if (better(kk[e], ki[e], kk[b], ki[b])) b = e;
-    float bk = kk[0];
-    int bi = ki[0];
-#pragma unroll
-    for (int e = 1; e < 4; ++e)
-      if (e == b) {
-        bk = kk[e];
-        bi = ki[e];
+    for (int u = 0; u < 4; ++u)
+      if (u == e) {
+        kk[u] = key;
+        ki[u] = i + u;
       }
-    const KeyIdx w = block_argmax(bk, bi, red);
-    if (t == 0) cand[j] = w;
+  });
+  wave_topk(kk, ki, a.k, list[t >> 6]);
+  supp = wave_sum(supp);
+  if (lane == 0) red_i[t >> 6] = supp;
+  __syncthreads();
+  if (t >= 64) return;
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (ki[e] == w.idx) {
-        kk[e] = -1.f;
-        ki[e] = NO_IDX;
-      }
+  for (int e = 0; e < 4; ++e) {  // 16 k <= 256 records, 4 a lane
+    const int j = lane + 64 * e;
+    const bool on = j < 16 * a.k;
+    kk[e] = on ? list[j / a.k][j % a.k].key : -1.f;
+    ki[e] = on ? list[j / a.k][j % a.k].idx : NO_IDX;
   }
-  if (t == 0) a.ws.csupp[(size_t)f * a.ws.C + c] = support;
+  wave_topk(kk, ki, a.k, a.ws.cand + ((size_t)f * a.ws.C + c) * SMP_MAXK);
+  if (t == 0) a.ws.csupp[(size_t)f * a.ws.C + c] = sum16(red_i);
 }
 
-// Per row: merge the chunks' candidates in chunk order; write min(k, support) tokens in draw
-// order and log q of each.
+// Per row: merge the chunks' candidates; write min(k, support) tokens in draw order and log q of each.
+// Wave w takes records 256 w .. of the row's C k (<= 4096), so up to 256 records need the first wave alone.
 __global__ __launch_bounds__(SMP_THREADS) void gumbel_merge_kernel(TopkArgs a) {
-  __shared__ KeyIdx red[16];
-  __shared__ int red_i[16];
+  __shared__ KeyIdx list[16][SMP_MAXK];
+  __shared__ KeyIdx best[SMP_MAXK];
   int F, base;
   frontier_rows(a.meta, a.level, a.rows, F, base);
-  const int f = blockIdx.x, t = threadIdx.x;
+  const int f = blockIdx.x, t = threadIdx.x, lane = t & 63, w = t >> 6;
   if (f >= F) return;
   const int C = a.ws.C;
   const int total = C * a.k;
   const float* q = a.q + (size_t)(base + f) * a.ldq;
-  int support = block_sum<int>(t < C ? a.ws.csupp[(size_t)f * C + t] : 0, red_i);
-  const int take = min(a.k, support);
-  // each thread holds up to 4 candidates (C * k <= 256 * 16 = 4096)
+  const int waves = (total + 255) / 256;  // <= 16: the launch has this many
   float kk[4];
   int ki[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int j = t * 4 + e;
-    if (j < total) {
-      const KeyIdx v = a.ws.cand[((size_t)f * C + j / a.k) * SMP_MAXK + j % a.k];
-      kk[e] = v.key;
-      ki[e] = v.idx;
-    } else {
-      kk[e] = -1.f;
-      ki[e] = NO_IDX;
+    const int j = 256 * w + lane + 64 * e;
+    const KeyIdx v = j < total ? a.ws.cand[((size_t)f * C + j / a.k) * SMP_MAXK + j % a.k] : KeyIdx{-1.f, NO_IDX};
+    kk[e] = v.key;
+    ki[e] = v.idx;
+  }
+  int supp = 0;
+  if (w == 0)
+    for (int u = lane; u < C; u += 64) supp += a.ws.csupp[(size_t)f * C + u];
+  if (waves > 1) {
+    wave_topk(kk, ki, a.k, list[w]);
+    __syncthreads();
+    if (w > 0) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int j = lane + 64 * e;
+      const bool on = j < waves * a.k;
+      kk[e] = on ? list[j / a.k][j % a.k].key : -1.f;
+      ki[e] = on ? list[j / a.k][j % a.k].idx : NO_IDX;
     }
   }
-  for (int r = 0; r < a.k; ++r) {
-    int tok = -1;
-    if (r < take) {
-      int b = 0;
-#pragma unroll
-      for (int e = 1; e < 4; ++e)
-        if (better(kk[e], ki[e], kk[b], ki[b])) b = e;
-      float bk = kk[0];
-      int bi = ki[0];
-#pragma unroll
-      for (int e = 1; e < 4; ++e)
-        if (e == b) {
-          bk = kk[e];
-          bi = ki[e];
-        }
-      const KeyIdx w = block_argmax(bk, bi, red);
-      tok = w.idx == NO_IDX ? -1 : w.idx;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (ki[e] == w.idx) {
-          kk[e] = -1.f;
-          ki[e] = NO_IDX;
-        }
-    }
-    if (t == 0) {
-      a.out_tok[f * a.k + r] = tok;
-      a.out_lp[f * a.k + r] = tok >= 0 ? logf(q[tok]) : 0.f;
-    }
+  const int take = min(a.k, wave_sum(supp));
+  wave_topk(kk, ki, a.k, best);  // one wave: its lanes run in step, lane 0's writes are in order
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  if (lane < a.k) {
+    const int tok = lane < take && best[lane].idx != NO_IDX ? best[lane].idx : -1;
+    a.out_tok[f * a.k + lane] = tok;
+    a.out_lp[f * a.k + lane] = tok >= 0 ? logf(q[tok]) : 0.f;
   }
 }
 
@@ -648,17 +806,21 @@ __global__ __launch_bounds__(SMP_THREADS) void draw_chunk_kernel(const float* __
   const U4 r = rng_block(rng, (uint32_t)(i >> 2), (uint32_t)row, TAG_DRAW);
   float best = -1.f;
   int bi = NO_IDX;
+  uint32_t on = 0;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    if (i + e < V && v[e] > 0.f) {
-      const float key = v[e] / exp1_from_bits(u4_get(r, e));
-      if (better(key, i + e, best, bi)) {
-        best = key;
-        bi = i + e;
-      }
+  for (int e = 0; e < 4; ++e) on |= (uint32_t)(i + e < V && v[e] > 0.f) << e;
+  for_active(on, [&](int e) {
+    const float key = get4(v, e) / exp1_from_bits(u4_get(r, e));
+    if (better(key, i + e, best, bi)) {
+      best = key;
+      bi = i + e;
     }
-  }
-  const KeyIdx w = block_argmax(best, bi, red);
+  });
+  KeyIdx w = wave_argmax(best, bi);
+  if ((t & 63) == 0) red[t >> 6] = w;
+  __syncthreads();
+  if (t >= 64) return;
+  w = argmax16(red);
   if (t == 0) ws.arg[(size_t)row * ws.C + c] = w;
 }
 
@@ -684,9 +846,14 @@ __global__ void draw_merge_kernel(int rows, SmpWs ws, int* __restrict__ out_tok)
 //             p_j = p_{j-1} otherwise,
 // and bonus[j] = the categorical draw from p_j (one shared Exp(1) vector per round: only one
 // state's draw is ever used, and which one is decided by the acceptance uniforms alone).
-// Pass j (one launch over all rows and chunks) produces the chunk partials of zr[j] and
-// bonus[j]; partials are combined by whoever needs them (the next pass, the walk), always by
-// the same wave reduction (combine_states), so every reader sees the same values.
+// The first launch over all rows and chunks produces the partials of bonus[0] and of state 1 (its
+// residual p - q0 needs no sums), pass j >= 2 those of zr[j] and bonus[j]; partials are combined by whoever
+// needs them (the next pass, the walk), always by the same wave reduction (combine_states), so every
+// reader sees the same values. The passes are bound by their chains of dependent loads (tree -> tokens ->
+// q0), not by bytes: the first one stores each row's child list for the others, loads the rows of P and Q
+// beside that chain, and the walk resolves every node at once, one wave each. us for 16 rows of 128256,
+// 3 children, before / after: pass 0 13.4 and pass 1 12.0 / first pass 11.4, pass j 12.0 / 8.4, walk
+// 8.4 / 6.6.
 struct AcceptArgs {
   SsdTree tree;
   const float* P;
@@ -703,12 +870,6 @@ struct AcceptArgs {
 constexpr int SMP_MAXNODES = 63;  // verify nodes (rows = nodes + 1 <= 64)
 
 __device__ __forceinline__ int verify_nodes(const SsdTree& t) { return min(t.vmeta[0], SMP_MAXNODES); }
-
-struct NodeKids {
-  int n;
-  int kid[SMP_MAXK];
-  int tok[SMP_MAXK];
-};
 
 __device__ __forceinline__ const float* q_row(const AcceptArgs& a, int cur) {
   return a.Q + (size_t)(cur < 0 ? 0 : 1 + a.tree.vorig[cur]) * a.ldq;
@@ -753,32 +914,6 @@ __device__ __forceinline__ void node_kids_block(const AcceptArgs& a, int cur, No
   __syncthreads();
 }
 
-// Wave reductions: a butterfly of exchanges, so every lane ends with the same value (each step adds
-// the same two partials on both lanes, and floating-point addition is commutative) and the order
-// of the additions is fixed.
-__device__ __forceinline__ double wave_sum_d(double v) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) v += __shfl_xor(v, o);
-  return v;
-}
-__device__ __forceinline__ int wave_sum_i(int v) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) v += __shfl_xor(v, o);
-  return v;
-}
-__device__ __forceinline__ KeyIdx wave_argmax(float k, int i) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const float ok = __shfl_xor(k, o);
-    const int oi = __shfl_xor(i, o);
-    if (better(ok, oi, k, i)) {
-      k = ok;
-      i = oi;
-    }
-  }
-  return KeyIdx{k, i};
-}
-
 struct StateScalars {
   double s0;
   int supp;
@@ -805,16 +940,16 @@ __device__ __forceinline__ void combine_states(const AcceptArgs& a, int r, const
     if (j <= upto)
       for (int c = lane; c < C; c += 64) z[j] += a.ws.zr[((size_t)r * (SMP_MAXK + 1) + j) * C + c];
   }
-  s0 = wave_sum_d(s0);
+  s0 = wave_sum(s0);
   s.s0 = s0;
-  s.supp = wave_sum_i(supp);
+  s.supp = wave_sum(supp);
   s.zr[0] = 0.f;
   s.zq[0] = 1.f;
   double zq = s0;
 #pragma unroll
   for (int j = 1; j <= SMP_MAXK; ++j) {
     if (j <= upto) {  // uniform
-      const double zj = wave_sum_d(z[j]);
+      const double zj = wave_sum(z[j]);
       s.zr[j] = zj > 0.0 ? (float)zj : 0.f;
       zq -= (double)q0[k.tok[j - 1]];
       s.zq[j] = (float)zq;
@@ -839,89 +974,115 @@ __device__ __forceinline__ float chain_p(float p0, float q0, int y, int j, const
   return pv;
 }
 
-// Pass 0: bonus draw from p_0 per chunk; q0's mass and support per chunk.
-__global__ __launch_bounds__(SMP_THREADS) void state0_kernel(AcceptArgs a) {
-  __shared__ KeyIdx red[16];
-  __shared__ double red_d[16];
+// Pass 0 and 1: the draws from p_0 and p_1 per chunk, the mass of p_1's residual, q0's mass and support.
+// One more workgroup per row (chunk index C) stores the row's child list.
+__global__ __launch_bounds__(SMP_THREADS) void state01_kernel(AcceptArgs a) {
+  __shared__ KeyIdx red0[16], red1[16];
+  __shared__ double red_s[16], red_z[16];
   __shared__ int red_i[16];
   __shared__ int sh_par[64], sh_rank[64], sh_pos[SMP_MAXK];
   __shared__ NodeKids kids;
   const int r = blockIdx.y, c = blockIdx.x, t = threadIdx.x;
-  if (r > verify_nodes(a.tree)) return;
   const int cur = r - 1;
-  node_kids_block(a, cur, kids, sh_par, sh_rank, sh_pos);
   const int i = c * SMP_CHUNK + t * 4;
-  float p[4];
-  load4_f32(a.P + (size_t)r * a.ldp, i, a.V, p);
+  float p[4], q[4] = {0.f, 0.f, 0.f, 0.f};
+  if (c < a.ws.C) load4_f32(a.P + (size_t)r * a.ldp, i, a.V, p);
+  const int vn = verify_nodes(a.tree);
+  if (r > vn) return;
+  if (c == a.ws.C) {
+    node_kids_block(a, cur, kids, sh_par, sh_rank, sh_pos);
+    if (t < (int)(sizeof(NodeKids) / 4)) ((int*)&a.ws.kids[r])[t] = ((const int*)&kids)[t];
+    return;
+  }
+  // a row without children in the tree has no draft row (its node may never have proposed)
+  if (__syncthreads_or(t < vn && a.max_kids > 0 && a.tree.vparents[t] == cur)) load4_f32(q_row(a, cur), i, a.V, q);
   const U4 rb = rng_block(a.rng, (uint32_t)(i >> 2), 0u, TAG_BONUS);
-  float best = -1.f;
-  int bi = NO_IDX;
+  float best0 = -1.f, best1 = -1.f;
+  int bi0 = NO_IDX, bi1 = NO_IDX, supp = 0;
+  double s0 = 0.0, zs = 0.0;
+  uint32_t on = 0;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    if (i + e < a.V && p[e] > 0.f) {
-      const float key = p[e] / exp1_from_bits(u4_get(rb, e));
-      if (better(key, i + e, best, bi)) {
-        best = key;
-        bi = i + e;
-      }
-    }
+    s0 += (double)q[e];
+    supp += q[e] > 0.f;
+    if (i + e < a.V) zs += (double)fmaxf(p[e] - q[e], 0.f);  // (p_0 - q_0)+
+    on |= (uint32_t)(i + e < a.V && p[e] > 0.f) << e;
   }
-  const KeyIdx w = block_argmax(best, bi, red);
-  double s0 = 0.0;
-  int supp = 0;
-  if (kids.n > 0) {
-    float q[4];
-    load4_f32(q_row(a, cur), i, a.V, q);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      s0 += (double)q[e];
-      supp += q[e] > 0.f;
+  for_active(on, [&](int e) {
+    const float pe = get4(p, e), res = fmaxf(pe - get4(q, e), 0.f);
+    const float ex = exp1_from_bits(u4_get(rb, e));
+    const float k0 = pe / ex, k1 = res / ex;
+    if (better(k0, i + e, best0, bi0)) {
+      best0 = k0;
+      bi0 = i + e;
     }
-    s0 = block_sum<double>(s0, red_d);
-    supp = block_sum<int>(supp, red_i);
+    if (res > 0.f && better(k1, i + e, best1, bi1)) {
+      best1 = k1;
+      bi1 = i + e;
+    }
+  });
+  KeyIdx w0 = wave_argmax(best0, bi0), w1 = wave_argmax(best1, bi1);
+  s0 = wave_sum(s0);
+  zs = wave_sum(zs);
+  supp = wave_sum(supp);
+  if ((t & 63) == 0) {
+    red0[t >> 6] = w0;
+    red1[t >> 6] = w1;
+    red_s[t >> 6] = s0;
+    red_z[t >> 6] = zs;
+    red_i[t >> 6] = supp;
   }
+  __syncthreads();
+  if (t >= 64) return;
+  w0 = argmax16(red0);
+  w1 = argmax16(red1);
   if (t == 0) {
     const int C = a.ws.C;
-    a.ws.bon[((size_t)r * (SMP_MAXK + 1) + 0) * C + c] = w;
-    a.ws.s0[(size_t)r * C + c] = s0;
-    a.ws.supp[(size_t)r * C + c] = supp;
+    a.ws.bon[((size_t)r * (SMP_MAXK + 1) + 0) * C + c] = w0;
+    // of a row without children, state 1 and q0's sums are not read
+    a.ws.bon[((size_t)r * (SMP_MAXK + 1) + 1) * C + c] = w1;
+    a.ws.zr[((size_t)r * (SMP_MAXK + 1) + 1) * C + c] = sum16(red_z);
+    a.ws.s0[(size_t)r * C + c] = sum16(red_s);
+    a.ws.supp[(size_t)r * C + c] = sum16(red_i);
   }
 }
 
-// Pass j >= 1: residual of state j-1 -> chunk partials of zr[j] and of the draw from p_j.
+// Pass j >= 2: residual of state j-1 -> chunk partials of zr[j] and of the draw from p_j.
 __global__ __launch_bounds__(SMP_THREADS) void statej_kernel(AcceptArgs a, int j) {
   __shared__ KeyIdx red[16];
   __shared__ double red_d[16];
-  __shared__ int sh_par[64], sh_rank[64], sh_pos[SMP_MAXK];
   __shared__ NodeKids kids;
   __shared__ StateScalars st;
   const int r = blockIdx.y, c = blockIdx.x, t = threadIdx.x;
   if (r > verify_nodes(a.tree)) return;
-  const int cur = r - 1;
-  node_kids_block(a, cur, kids, sh_par, sh_rank, sh_pos);
-  if (kids.n < j) return;  // uniform: this node has fewer children
-  const float* q0 = q_row(a, cur);
-  if (t < 64) combine_states(a, r, q0, kids, j - 1, st);  // wave 0; its lanes store the same values
-  __syncthreads();
+  const int n = a.ws.kids[r].n;
+  const float* q0 = q_row(a, r - 1);
+  if (n < j) return;  // uniform: this node has fewer children
   const int i = c * SMP_CHUNK + t * 4;
   float p[4], q[4];
   load4_f32(a.P + (size_t)r * a.ldp, i, a.V, p);
   load4_f32(q0, i, a.V, q);
+  if (t < (int)(sizeof(NodeKids) / 4)) ((int*)&kids)[t] = ((const int*)&a.ws.kids[r])[t];
   const U4 rb = rng_block(a.rng, (uint32_t)(i >> 2), 0u, TAG_BONUS);
+  __syncthreads();
+  if (t < 64) combine_states(a, r, q0, kids, j - 1, st);  // wave 0; its lanes store the same values
+  __syncthreads();
   double zs = 0.0;
   float best = -1.f;
   int bi = NO_IDX;
+  // p_0(y) = 0 leaves no residual in any state as long as the draft mass left is positive (rounding can
+  // leave it at or below 0 once what remains is under 1e-16 of it)
+  const bool all = !(st.zq[j - 1] > 0.f);
+  uint32_t on = 0;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
+  for (int e = 0; e < 4; ++e) on |= (uint32_t)(i + e < a.V && (p[e] > 0.f || all)) << e;
+  for_active(on, [&](int e) {
     const int y = i + e;
-    if (y >= a.V) continue;
-    const float pprev = chain_p(p[e], q[e], y, j - 1, st.zr, st.zq, kids.tok);
-    float qprev = q[e];
-    if (j - 1 > 0) {
-      bool rj = false;
-      for (int u = 0; u < j - 1; ++u) rj |= kids.tok[u] == y;
-      qprev = rj ? 0.f : q[e] / st.zq[j - 1];
-    }
+    const float qe = get4(q, e);
+    const float pprev = chain_p(get4(p, e), qe, y, j - 1, st.zr, st.zq, kids.tok);
+    bool rj = false;
+    for (int u = 0; u < j - 1; ++u) rj |= kids.tok[u] == y;
+    const float qprev = rj ? 0.f : qe / st.zq[j - 1];
     const float res = fmaxf(pprev - qprev, 0.f);
     zs += (double)res;
     if (res > 0.f) {
@@ -931,82 +1092,100 @@ __global__ __launch_bounds__(SMP_THREADS) void statej_kernel(AcceptArgs a, int j
         bi = y;
       }
     }
+  });
+  zs = wave_sum(zs);
+  KeyIdx w = wave_argmax(best, bi);
+  if ((t & 63) == 0) {
+    red_d[t >> 6] = zs;
+    red[t >> 6] = w;
   }
-  zs = block_sum<double>(zs, red_d);
-  const KeyIdx w = block_argmax(best, bi, red);
+  __syncthreads();
+  if (t >= 64) return;
+  w = argmax16(red);
   if (t == 0) {
     const int C = a.ws.C;
-    a.ws.zr[((size_t)r * (SMP_MAXK + 1) + j) * C + c] = zs;
+    a.ws.zr[((size_t)r * (SMP_MAXK + 1) + j) * C + c] = sum16(red_d);
     a.ws.bon[((size_t)r * (SMP_MAXK + 1) + j) * C + c] = w;
   }
 }
 
 // The walk of sample_verify over the state scalars, then the same bookkeeping as the greedy
-// walk: result = [n_new, tokens...], compaction sources, next root token. One wave: every lane
-// walks the same path with the same values (the child lists, the state sums and the bonus merge
-// are wave-wide operations), lane 0 writes the result.
-__global__ __launch_bounds__(64) void sample_walk_kernel(AcceptArgs a, int committed, int* result, int* keep_src,
-                                                        int* n_keep, int* root_token) {
-  __shared__ int sh_par[64], sh_rank[64], sh_pos[SMP_MAXK];
-  __shared__ NodeKids kids;
-  const int lane = threadIdx.x;
-  const int C = a.ws.C;
-  int cur = -1, n_acc = 0, bonus = 0;
-  int rej[SMP_MAXK];
-  StateScalars s;
-  for (int step = 0; step <= SMP_MAXDEPTH; ++step) {
-    const int r = cur + 1;
-    if (r >= a.rows) break;  // a tree larger than the launch's rows (the engine never makes one)
-    node_kids_block(a, cur, kids, sh_par, sh_rank, sh_pos);
+// walk: result = [n_new, tokens...], compaction sources, next root token. What happens at a node --
+// which child is accepted, or which bonus token is drawn -- depends on that node's row alone, so wave w
+// resolves rows w, w + 16, ... (all lanes with the same values; the state sums and the bonus merge are
+// wave-wide operations), and one thread then follows the path.
+__global__ __launch_bounds__(SMP_THREADS) void sample_walk_kernel(AcceptArgs a, int committed, int* result,
+                                                                 int* keep_src, int* n_keep, int* root_token) {
+  __shared__ int next[SMP_MAXNODES + 1], drawn[SMP_MAXNODES + 1], tok_sh[SMP_MAXNODES + 1];
+  __shared__ NodeKids kids_sh[16];
+  __shared__ StateScalars st_sh[16];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int C = a.ws.C, n_rows = min(verify_nodes(a.tree) + 1, a.rows);
+  if (threadIdx.x < n_rows - 1) tok_sh[threadIdx.x] = a.tree.vtokens[threadIdx.x];
+  NodeKids& kids = kids_sh[wv];  // this wave's own, read back by the lanes that wrote them or in step with them
+  StateScalars& s = st_sh[wv];
+  for (int r = wv; r < n_rows; r += 16) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (lane < (int)(sizeof(NodeKids) / 4)) ((int*)&kids)[lane] = ((const int*)&a.ws.kids[r])[lane];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const int kn = kids.n;
-    const float* q0 = q_row(a, cur);
+    const float* q0 = q_row(a, r - 1);
     const float* p = a.P + (size_t)r * a.ldp;
-    s.supp = 0;
-    s.zr[0] = 0.f;
-    s.zq[0] = 1.f;
     if (kn > 0) combine_states(a, r, q0, kids, kn, s);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // lane i: child i's p and q0
+    const int x_l = lane < kn ? kids.tok[lane] : 0;
+    const float p_l = lane < kn ? p[x_l] : 0.f, q_l = lane < kn ? q0[x_l] : 0.f;
     int chosen = -1, j = 0;
-    for (int i = 0; i < kn; ++i) {
-      const int x = kids.tok[i];
-      const float q0x = q0[x];
-      const float pj = chain_p(p[x], q0x, x, j, s.zr, s.zq, rej);
+    for (int i = 0; i < kn; ++i) {  // j == i: the children before i were rejected
+      const int x = __shfl(x_l, i);
+      const float q0x = __shfl(q_l, i);
+      const float pj = chain_p(__shfl(p_l, i), q0x, x, j, s.zr, s.zq, kids.tok);
       const float qj = j == 0 ? q0x : q0x / s.zq[j];
       const double u = uniform_from_bits(rng_block(a.rng, (uint32_t)j, (uint32_t)r, TAG_ACCEPT).x);
       if (u < (double)fminf(1.f, pj / qj)) {
         chosen = kids.kid[i];
         break;
       }
-      rej[j] = x;
       ++j;
       if (j >= s.supp) break;  // no draft mass left
     }
+    KeyIdx b{-1.f, NO_IDX};
     if (chosen < 0) {
       int jj = j;
       while (jj > 0 && !(s.zr[jj] > 0.f)) --jj;  // p_j == p_{j-1} when the residual had no mass
       // the categorical draw from p_jj: the best of the chunks' records (a strict order on
       // (key, column), so any merge order gives the same record)
       const KeyIdx* part = a.ws.bon + ((size_t)r * (SMP_MAXK + 1) + jj) * C;
-      KeyIdx b{-1.f, NO_IDX};
       for (int c = lane; c < C; c += 64)
         if (better(part[c].key, part[c].idx, b.key, b.idx)) b = part[c];
       b = wave_argmax(b.key, b.idx);
-      bonus = b.idx == NO_IDX ? 0 : b.idx;
-      break;
     }
     if (lane == 0) {
-      result[1 + n_acc] = a.tree.vtokens[chosen];
-      keep_src[1 + n_acc] = committed + 1 + chosen;
+      next[r] = chosen;
+      drawn[r] = b.idx == NO_IDX ? 0 : b.idx;
     }
+  }
+  __syncthreads();
+  if (threadIdx.x) return;
+  int cur = -1, n_acc = 0, bonus = 0;
+  for (int step = 0; step <= SMP_MAXDEPTH; ++step) {
+    const int r = cur + 1;
+    if (r >= n_rows) break;  // a tree larger than the launch's rows (the engine never makes one)
+    if (next[r] < 0) {
+      bonus = drawn[r];
+      break;
+    }
+    cur = next[r];
+    result[1 + n_acc] = tok_sh[cur];
+    keep_src[1 + n_acc] = committed + 1 + cur;
     ++n_acc;
-    cur = chosen;
   }
-  if (lane == 0) {
-    result[1 + n_acc] = bonus;
-    result[0] = n_acc + 1;
-    keep_src[0] = committed;
-    *n_keep = n_acc + 1;
-    *root_token = bonus;
-  }
+  result[1 + n_acc] = bonus;
+  result[0] = n_acc + 1;
+  keep_src[0] = committed;
+  *n_keep = n_acc + 1;
+  *root_token = bonus;
 }
 
 // ------------------------------------------------------ batched acceptance trials
@@ -1016,7 +1195,7 @@ __global__ __launch_bounds__(64) void sample_walk_kernel(AcceptArgs a, int commi
 // unpruned with branch[d] children per node at level d, numbered level by level (level L node with
 // in-level index f has children start[L + 1] + f * branch[L + 1] + i, i = draw order). Each trial
 // draws only the children on its walk; every draw and decision uses the engine's streams,
-// counters and formulas (gumbel_chunk / state0 / statej / sample_walk above): Gumbel keys
+// counters and formulas (gumbel_chunk / state01 / statej / sample_walk above): Gumbel keys
 // q / Exp(1) from the PROPOSE stream at (column / 4, f | level << 16), acceptance uniforms at
 // (rejections, row), residual states through chain_p, the bonus race on the unnormalised
 // residual at (column / 4, 0). Sums run over each row's support list (columns where P or Q is
@@ -1078,8 +1257,8 @@ __global__ __launch_bounds__(256) void accept_trials_kernel(TrialArgs a) {
         s0 += (double)qv;
         supp += qv > 0.f;
       }
-      s0 = wave_sum_d(s0);
-      supp = wave_sum_i(supp);
+      s0 = wave_sum(s0);
+      supp = wave_sum(supp);
       int take = min(k, supp);
       int tok[SMP_MAXK];
       for (int c = 0; c < take; ++c) {
@@ -1129,7 +1308,7 @@ __global__ __launch_bounds__(256) void accept_trials_kernel(TrialArgs a) {
           const float pprev = chain_p(p[y], q[y], y, j - 1, zr, zq, rej);
           z += (double)fmaxf(pprev - trial_qprev(q[y], y, j, zq, rej), 0.f);
         }
-        z = wave_sum_d(z);
+        z = wave_sum(z);
         zr[j] = z > 0.0 ? (float)z : 0.f;
         if (j >= supp) break;  // no draft mass left
       }
@@ -1384,7 +1563,7 @@ SSD_API int ssd_gumbel_topk(const float* probs, int64_t ldp, int rows, int V, in
   if (int rc = carve(ws, ws_bytes, rows, V, &w, "gumbel_topk")) return rc;
   TopkArgs a{probs, ldp, rows, V, k, tree_meta, level, make_rng(seed, counter), out_tok, out_lp, w};
   SSD_LAUNCH(gumbel_chunk_kernel, dim3(w.C, rows), dim3(SMP_THREADS), 0, stream, a);
-  SSD_LAUNCH(gumbel_merge_kernel, dim3(rows), dim3(SMP_THREADS), 0, stream, a);
+  SSD_LAUNCH(gumbel_merge_kernel, dim3(rows), dim3(64 * ((w.C * k + 255) / 256)), 0, stream, a);
   return check_launch("gumbel_topk");
 }
 
@@ -1444,10 +1623,10 @@ SSD_API int ssd_accept_sample(const SsdTree* tree, const float* P, int64_t ldp, 
   SmpWs w;
   if (int rc = carve(ws, ws_bytes, rows, V, &w, "accept_sample")) return rc;
   AcceptArgs a{*tree, P, ldp, Q, ldq, V, rows, max_kids, make_rng(seed, counter), w};
-  SSD_LAUNCH(state0_kernel, dim3(w.C, rows), dim3(SMP_THREADS), 0, stream, a);
-  for (int j = 1; j <= max_kids; ++j)
+  SSD_LAUNCH(state01_kernel, dim3(w.C + 1, rows), dim3(SMP_THREADS), 0, stream, a);
+  for (int j = 2; j <= max_kids; ++j)
     SSD_LAUNCH(statej_kernel, dim3(w.C, rows), dim3(SMP_THREADS), 0, stream, a, j);
-  SSD_LAUNCH(sample_walk_kernel, dim3(1), dim3(64), 0, stream, a, committed, result, keep_src, n_keep,
+  SSD_LAUNCH(sample_walk_kernel, dim3(1), dim3(SMP_THREADS), 0, stream, a, committed, result, keep_src, n_keep,
                      root_token);
   return check_launch("accept_sample");
 }
