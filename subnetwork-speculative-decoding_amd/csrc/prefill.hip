@@ -19,7 +19,7 @@
 //   q/k/v 183 (227): 0.52 of the MFMA peak at gate/up and down. Taking the loads out of the loop gives
 //   down 230 us: the loads' path through L2 bounds the large tiles; small ones are bound by a step's
 //   chain of barrier, MFMAs and LDS reads.
-// * prefill_attention_kernel: causal flash attention, one wave per (q head, 32 tokens), K/V read
+// * prefill_attention_kernel: causal flash attention, one wave per (q head, 16 or 32 tokens), K/V read
 //   in the cache's 64-slot MFMA-operand blocks; S^T = K Q^T and O^T = V^T P^T on MFMA with the
 //   running max / sum rescaled per 64-key block.
 // * ssd_prefill: the whole target forward for one chunk of prompt rows in one C call.
@@ -604,32 +604,32 @@ __device__ __forceinline__ float pf_sum_lanes(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-constexpr int PF_TOK = 32;  // tokens per wave (two 16-row tiles)
-
-// Per-wave state of the causal attention: the query fragments of two 16-row tiles, their running
-// max / sum and output accumulators, and each lane's last attended key.
-template <int HD>
+// Per-wave state of the causal attention: the query fragments of NT 16-row tiles (16 NT tokens), their
+// running max / sum and output accumulators, and each lane's last attended key.
+template <int HD, int NT>
 struct PfAttnState {
-  static constexpr int KS = HD / 32, DT = HD / 16, NT = PF_TOK / 16;
+  static constexpr int KS = HD / 32, DT = HD / 16;
   u32x4_t qf[NT][KS];
   float m_run[NT], l_run[NT];
   f32x4_t o[NT][DT];
   int lim[NT];
 };
 
-// One 64-key block b for both row tiles. K / V fragments come from `ck` / `cv` (the block in LDS,
+// One 64-key block b for the wave's row tiles. K / V fragments come from `ck` / `cv` (the block in LDS,
 // SHARED) or from the cache rows `kb` / `vb`; with SHARED the copy of block b + 1 into `nk` / `nv`
 // is issued first. The LDS pointers are restrict, so the compiler sees that the fragment reads do
-// not touch the buffer being filled and does not wait for that copy before them.
-template <int HD, bool SHARED>
-__device__ __forceinline__ void pf_attend_block(PfAttnState<HD>& st, int b, int n_blk, int full_blk, int last,
-                                                float scale_log2, int lane, const bf16_t* kb, const bf16_t* vb,
-                                                const u32x4_t* ksrc, const u32x4_t* vsrc,
+// not touch the buffer being filled and does not wait for that copy before them. MASKED: the block may
+// hold keys past a row's own or past the tile's last (the one or two last blocks of a tile; the other
+// blocks need 200 vector instructions without the masks, 340 with them: 32 heads of 4096 tokens 173 -> 143 us).
+template <int HD, bool SHARED, int NT, bool MASKED>
+__device__ __forceinline__ void pf_attend_block(PfAttnState<HD, NT>& st, int b, int n_blk, int last,
+                                                float scale_log2, int lane, int w, const bf16_t* kb, const bf16_t* vb,
+                                                const char* ksrc, const char* vsrc,
                                                 const lds_u32x4* __restrict__ ck, const lds_u32x4* __restrict__ cv,
                                                 lds_u32x4* __restrict__ nk, lds_u32x4* __restrict__ nv) {
-  constexpr int KS = HD / 32, DT = HD / 16, NT = PF_TOK / 16;
+  constexpr int KS = HD / 32, DT = HD / 16;
   constexpr int PIECES = 64 * HD / 8;  // 16-byte pieces of one block's K (and of its V^T)
-  const int g = lane >> 4, w = threadIdx.x >> 6;
+  const int g = lane >> 4;
   if constexpr (SHARED) {
     // this block's copy landed (the only loads in flight: an explicit wait, since a workgroup
     // barrier does not wait for global-to-LDS loads) and every wave is done with the buffer the next
@@ -638,14 +638,16 @@ __device__ __forceinline__ void pf_attend_block(PfAttnState<HD>& st, int b, int 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (b + 1 < n_blk) {
-      // wave w, load i copies pieces 256 i + 64 w + lane of block b + 1's K and V^T
-      const size_t off = (size_t)(b + 1) * PIECES + 64 * w;
+      // wave w, load i copies pieces 256 i + 64 w + lane of block b + 1's K and V^T (scalar pointer plus
+      // a 32-bit lane offset)
+      const size_t off = ((size_t)(b + 1) * PIECES + 64 * w) * 16;
+      const uint32_t l16 = lane * 16;
 #pragma unroll
       for (int i = 0; i < PIECES / 256; ++i) {
-        __builtin_amdgcn_global_load_lds((const void*)(ksrc + off + 256 * i),
-                                         (__attribute__((address_space(3))) void*)(nk + 256 * i + 64 * w), 16, 0, 0);
-        __builtin_amdgcn_global_load_lds((const void*)(vsrc + off + 256 * i),
-                                         (__attribute__((address_space(3))) void*)(nv + 256 * i + 64 * w), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const void*)(ksrc + off + 4096 * i + l16), (lds_void*)(nk + 256 * i + 64 * w), 16,
+                                         0, 0);
+        __builtin_amdgcn_global_load_lds((const void*)(vsrc + off + 4096 * i + l16), (lds_void*)(nv + 256 * i + 64 * w), 16,
+                                         0, 0);
       }
     }
   }
@@ -682,7 +684,7 @@ __device__ __forceinline__ void pf_attend_block(PfAttnState<HD>& st, int b, int 
       vf[dt][1] = *(const u32x4_t*)(vb + (size_t)b * 64 * HD + (dt * 2 + 1) * 512);
     }
   }
-  if (b == n_blk - 1) {
+  if (MASKED && b == n_blk - 1) {
     // slots past the tile's last key hold whatever the cache held (not yet written): their
     // probabilities are 0, and 0 * V must stay 0, so V is zeroed there. Lane (g, i) of V tile
     // (dt, c) holds slots 64 b + 32 c + 8 g .. + 8.
@@ -697,7 +699,6 @@ __device__ __forceinline__ void pf_attend_block(PfAttnState<HD>& st, int b, int 
       for (int dt = 0; dt < DT; ++dt) vf[dt][c] &= keep;
     }
   }
-  const bool masked = b >= full_blk;
 #pragma unroll
   for (int rt = 0; rt < NT; ++rt) {
     // Softmax in base 2 with the score scale folded into the exponent: p = 2^(s c - m), m a running
@@ -711,7 +712,7 @@ __device__ __forceinline__ void pf_attend_block(PfAttnState<HD>& st, int b, int 
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         float v = s[rt][kt][e];
-        if (masked && b * 64 + pf_perm_key(kt, 4 * g + e) > st.lim[rt]) v = -INFINITY;
+        if (MASKED && b * 64 + pf_perm_key(kt, 4 * g + e) > st.lim[rt]) v = -INFINITY;
         sv[kt * 4 + e] = v;
         mx = fmaxf(mx, v);
       }
@@ -731,7 +732,7 @@ __device__ __forceinline__ void pf_attend_block(PfAttnState<HD>& st, int b, int 
         pw[kt >> 1][(kt & 1) * 2 + e / 2] = pack_bf16x2(p0, p1);
       }
     l = pf_sum_lanes(l);
-    st.l_run[rt] = st.l_run[rt] * alpha + l;
+    st.l_run[rt] = fmaf(st.l_run[rt], alpha, l);  // spelled out: the masked and the plain instance must agree
     st.m_run[rt] = m_use;
     if (__builtin_amdgcn_ballot_w64(grow)) {  // wave-uniform: multiplying by alpha = 1 is exact
 #pragma unroll
@@ -751,16 +752,20 @@ __device__ __forceinline__ void pf_attend_block(PfAttnState<HD>& st, int b, int 
 // cache layout kept) one block ahead of its use, and the waves read their MFMA fragments from there;
 // otherwise every wave loads its block's K and V straight into registers when it needs them. The
 // fragments and their order are the same either way, so the outputs are bit-identical.
-template <int HD, bool SHARED>
+// NT: 16-row tiles per wave. Two halve the K / V fragment reads per row; one gives a short prompt twice
+// the workgroups, each with half the work per block (a block then takes its chain of barrier, LDS reads,
+// MFMAs and softmax, not its throughput): 32 heads of 512 tokens 18.3 us with two, 11.0 with one; 100
+// tokens 8.1 and 5.6.
+template <int HD, bool SHARED, int NT>
 __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const bf16_t* __restrict__ Q, int64_t ldq, int M,
                                                                    int pos0, int heads, int kv_heads,
                                                                    const bf16_t* __restrict__ Kc,
                                                                    const bf16_t* __restrict__ Vt, int64_t max_len,
                                                                    float scale_log2, bf16_t* __restrict__ out,
                                                                    int64_t ldo, int n_tt) {
-  constexpr int KS = HD / 32, DT = HD / 16, NT = PF_TOK / 16;
+  constexpr int KS = HD / 32, DT = HD / 16, TOK = 16 * NT;
   constexpr int PIECES = 64 * HD / 8;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 15, g = lane >> 4;
   const int n_hg = (heads + 3) / 4;
   // the longest token tiles first (their rows attend the most keys)
@@ -768,14 +773,14 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const bf16_t*
   const int h = ((int)blockIdx.x % n_hg) * 4 + w;
   if (!SHARED && h >= heads) return;  // SHARED launches have heads % 4 == 0 (no wave leaves early)
   const int kvh = h / (heads / kv_heads);
-  const int t0 = tt * PF_TOK;
+  const int t0 = tt * TOK;
   const bf16_t* kb = Kc + (size_t)kvh * max_len * HD + lane * 8;
   const bf16_t* vb = Vt + (size_t)kvh * max_len * HD + lane * 8;
-  // this kv head's blocks as 16-byte pieces (per lane) for the LDS copies
-  const u32x4_t* ksrc = (const u32x4_t*)(Kc + (size_t)kvh * max_len * HD) + lane;
-  const u32x4_t* vsrc = (const u32x4_t*)(Vt + (size_t)kvh * max_len * HD) + lane;
+  // this kv head's blocks for the LDS copies
+  const char* ksrc = (const char*)(Kc + (size_t)kvh * max_len * HD);
+  const char* vsrc = (const char*)(Vt + (size_t)kvh * max_len * HD);
 
-  PfAttnState<HD> st;
+  PfAttnState<HD, NT> st;
 #pragma unroll
   for (int rt = 0; rt < NT; ++rt) {
     const int tok = min(t0 + rt * 16 + j, M - 1);
@@ -788,9 +793,9 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const bf16_t*
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) st.o[rt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  const int last = pos0 + min(t0 + PF_TOK, M) - 1;  // the tile's last attended key
+  const int last = pos0 + min(t0 + TOK, M) - 1;  // the tile's last attended key
   const int n_blk = last / 64 + 1;
-  const int full_blk = (pos0 + t0) / 64;  // blocks every row of the tile attends entirely
+  const int full_blk = min((pos0 + t0) / 64, n_blk - 1);  // blocks every row of the tile attends entirely
 
   // two K / V^T buffers (SHARED): blocks alternate between them
   constexpr int BUF = SHARED ? PIECES : 1;
@@ -799,19 +804,32 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const bf16_t*
   if constexpr (SHARED) {
 #pragma unroll
     for (int i = 0; i < PIECES / 256; ++i) {
-      __builtin_amdgcn_global_load_lds((const void*)(ksrc + 256 * i + 64 * w),
-                                       (__attribute__((address_space(3))) void*)((lp)kA + 256 * i + 64 * w), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((const void*)(vsrc + 256 * i + 64 * w),
-                                       (__attribute__((address_space(3))) void*)((lp)vA + 256 * i + 64 * w), 16, 0, 0);
+      const size_t off = (size_t)(256 * i + 64 * w) * 16;
+      __builtin_amdgcn_global_load_lds((const void*)(ksrc + off + (uint32_t)lane * 16),
+                                       (lds_void*)((lp)kA + 256 * i + 64 * w), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((const void*)(vsrc + off + (uint32_t)lane * 16),
+                                       (lds_void*)((lp)vA + 256 * i + 64 * w), 16, 0, 0);
     }
   }
-  // blocks in pairs: each instance of the body reads one buffer and fills the other
-  for (int b = 0; b < n_blk; b += 2) {
-    pf_attend_block<HD, SHARED>(st, b, n_blk, full_blk, last, scale_log2, lane, kb, vb, ksrc, vsrc, (lp)kA, (lp)vA,
-                                (lp)kB, (lp)vB);
-    if (b + 1 < n_blk)
-      pf_attend_block<HD, SHARED>(st, b + 1, n_blk, full_blk, last, scale_log2, lane, kb, vb, ksrc, vsrc, (lp)kB,
-                                  (lp)vB, (lp)kA, (lp)vA);
+  // each instance of the body reads one buffer and fills the other
+  auto even = [&](auto masked, int b) {
+    pf_attend_block<HD, SHARED, NT, decltype(masked)::value>(st, b, n_blk, last, scale_log2, lane, w, kb, vb, ksrc, vsrc,
+                                                             (lp)kA, (lp)vA, (lp)kB, (lp)vB);
+  };
+  auto odd = [&](auto masked, int b) {
+    pf_attend_block<HD, SHARED, NT, decltype(masked)::value>(st, b, n_blk, last, scale_log2, lane, w, kb, vb, ksrc, vsrc,
+                                                             (lp)kB, (lp)vB, (lp)kA, (lp)vA);
+  };
+  using yes_t = std::integral_constant<bool, true>;
+  using no_t = std::integral_constant<bool, false>;
+  int b = 0;
+  for (; b + 1 < full_blk; b += 2) {
+    even(no_t{}, b);
+    odd(no_t{}, b + 1);
+  }
+  for (; b < n_blk; b += 2) {  // at most one block more that every row attends entirely, then the masked ones
+    even(yes_t{}, b);
+    if (b + 1 < n_blk) odd(yes_t{}, b + 1);
   }
   // lane (g, j) of o[rt][dt] holds dims 16 dt + 4 g + e of row j
 #pragma unroll
@@ -1022,27 +1040,34 @@ SSD_API int ssd_prefill_attention_bf16(const uint16_t* q, int64_t ldq, int M, in
       ((uintptr_t)vt_cache & 15) || ldo % 4 || ((uintptr_t)out & 7))
     return set_error(SSD_EINVAL, "prefill attention: rows [%d, %d) vs cache %lld, or misaligned operands", pos0,
                      pos0 + M, (long long)max_len);
-  const int n_tt = (M + PF_TOK - 1) / PF_TOK;
-  const dim3 grid((unsigned)(n_tt * ((heads + 3) / 4))), block(256);
+  // one 16-row tile per wave while that leaves at most two workgroups per CU
+  const int n_hg = (heads + 3) / 4;
+  const bool small = (int64_t)((M + 15) / 16) * n_hg <= 512;
+  const int tok = small ? 16 : 32, n_tt = (M + tok - 1) / tok;
+  const dim3 grid((unsigned)(n_tt * n_hg)), block(256);
   const float sl2 = scale * 1.4426950408889634f;
   // a workgroup's four waves share one kv head's K/V when 4 divides the q heads per kv head
   const bool shared = (heads / kv_heads) % 4 == 0;
-#define PF_ATT(D, SH)                                                                                         \
-  SSD_LAUNCH((prefill_attention_kernel<D, SH>), grid, block, 0, stream, (const bf16_t*)q, ldq, M, pos0, heads, \
+#define PF_ATT_NT(D, SH, NT)                                                                                       \
+  SSD_LAUNCH((prefill_attention_kernel<D, SH, NT>), grid, block, 0, stream, (const bf16_t*)q, ldq, M, pos0, heads, \
              kv_heads, (const bf16_t*)k_cache, (const bf16_t*)vt_cache, max_len, sl2, (bf16_t*)out, ldo, n_tt)
+#define PF_ATT(D, SH)               \
+  if (small) PF_ATT_NT(D, SH, 1);   \
+  else PF_ATT_NT(D, SH, 2)
   switch (head_dim) {
     case 64:
-      if (shared) PF_ATT(64, true);
-      else PF_ATT(64, false);
+      if (shared) { PF_ATT(64, true); }
+      else { PF_ATT(64, false); }
       break;
     case 128:
-      if (shared) PF_ATT(128, true);
-      else PF_ATT(128, false);
+      if (shared) { PF_ATT(128, true); }
+      else { PF_ATT(128, false); }
       break;
     default:
       return set_error(SSD_EINVAL, "prefill attention: head_dim %d unsupported (64, 128)", head_dim);
   }
 #undef PF_ATT
+#undef PF_ATT_NT
   return check_launch("prefill_attention");
 }
 

@@ -99,3 +99,25 @@ def test_rows_far_apart_equal_contiguous_rows():
     ops.prefill_gemm(x, m, wp, grp, n, k, a, residual=res)
     ops.prefill_gemm(far, m, wp, grp, n, k, b, residual=res)
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("heads,kv,hd", [(32, 8, 128), (32, 8, 64), (6, 3, 128)])
+def test_attention_rows_do_not_depend_on_the_tile(heads, kv, hd):
+    """A call with many rows gives each wave 32 tokens, one with few 16, and a row's block is masked or not
+    depending on its tile: the same rows in calls of other sizes and starts have the same bits."""
+    from ssd import ops
+
+    m = 128 * (32 // ((heads + 3) // 4)) + 70  # past the line between the two
+    cap = (m + 63) // 64 * 64 + 64
+    q = _rand(m, heads * hd, seed=9)
+    k, v = _rand(kv, cap, hd, seed=10), _rand(kv, cap, hd, seed=11)
+    k[:, m:] = float("nan")
+    v[:, m:] = float("nan")
+    kd, vd = ops.kv_tile(k, "k"), ops.kv_tile(v, "v")
+    ref = torch.zeros(m, heads * hd, dtype=torch.bfloat16, device=DEV)
+    ops.prefill_attention(q, m, 0, heads, kv, hd, kd, vd, cap, ref)
+    assert torch.isfinite(ref.float()).all()
+    for r0, n in ((0, 16), (0, 65), (37, 128), (64, 17), (100, 200), (m - 33, 33)):
+        out = torch.zeros(n, heads * hd, dtype=torch.bfloat16, device=DEV)
+        ops.prefill_attention(q[r0:r0 + n], n, r0, heads, kv, hd, kd, vd, cap, out)
+        assert torch.equal(out, ref[r0:r0 + n]), (r0, n)
