@@ -42,11 +42,15 @@ struct GemmLds {
   float rn[CT * 16];     // per-row rsqrt(mean(x^2) + eps)
 };
 
-// X staged through LDS (gemm_kernel<..., XS = true>): K = 4096 (8 rounds of 16 k-blocks), 8 waves.
-// Each round's rows are copied memory -> LDS by DMA as whole 1 KiB row segments (full 128-byte
-// lines, once per workgroup) instead of each wave loading its 64-byte row pieces itself; rows are
-// XS_ROW bytes apart so the 8 lanes a b128 read serves at a time fall in different banks.
-constexpr int XS_ROUNDS = 8, XS_SLOTS = 2, XS_AHEAD = 3, XS_ROW = 16 * 64 + 16;
+// X staged through LDS (gemm_kernel<..., XR = K / 512>): K = 2048, 4096 or 8192 (rounds of 16 k-blocks), 8
+// waves. Each round's rows are loaded as whole 1 KiB row segments (full 128-byte lines, once per
+// workgroup) instead of each wave loading its 64-byte row pieces itself; rows are XS_ROW bytes apart so
+// the 8 lanes a b128 read serves at a time fall in different banks. A workgroup reads all of X, as many
+// bytes as its weights or more, at the ~80 GB/s of a CU's load path, which is what bounds these calls:
+// pieces of half lines cost twice. us direct / staged: 8B q/k/v at 40 and 64 rows 17.7 / 15.2 and 24.1 / 17.0,
+// o 15.0 / 11.4 and 21.5 / 13.9; 70B q/k/v at 1, 25 and 64 rows 32.7 / 28.2, 47.3 / 32.7 and 83.2 / 41.7 (with
+// four tiles a workgroup, see plan_for). Loads run three rounds ahead, fewer where registers are short.
+constexpr int XS_SLOTS = 2, XS_ROW = 16 * 64 + 16;
 
 template <int KS, int NSUB, int CT, bool XS>
 union GemmSmem {
@@ -54,8 +58,11 @@ union GemmSmem {
   unsigned char ring[XS ? XS_SLOTS * CT * 16 * XS_ROW : 16];
 };
 
-template <int CT, int NSUB, int KS, int U, int EPI, int NORM, bool XS = false>
+template <int CT, int NSUB, int KS, int U, int EPI, int NORM, int XR = 0>
 __global__ __launch_bounds__(64 * KS) void gemm_kernel(GemmArgs a) {
+  constexpr bool XS = XR > 0;
+  constexpr int XS_ROUNDS = XR;
+  constexpr int XS_AHEAD = CT * (NSUB + 2) <= 8 ? 3 : CT * (NSUB + 2) <= 18 ? 2 : 1;  // rounds of loads in registers
   static_assert(!XS || KS == 8, "the staged path deals 16 k-blocks per round to 8 waves");
   __shared__ GemmSmem<KS, NSUB, CT, XS> smem;
   auto& lds = smem.g;
@@ -173,6 +180,11 @@ __global__ __launch_bounds__(64 * KS) void gemm_kernel(GemmArgs a) {
       }
       // slot (r + 1) % 2 last held round r - 1, which every wave finished before this barrier
       if (r + 1 < XS_ROUNDS) stage(r + 1);
+      if constexpr (NORM && CT * (NSUB + 2) > 8) {
+        // registers are short: the round's sums are finished here, not with its fragments kept for later
+#pragma unroll
+        for (int c = 0; c < CT; ++c) asm volatile("" : "+v"(ss[c]));
+      }
     }
     __syncthreads();  // the ring is reused for the partial sums below
   } else {
@@ -791,7 +803,9 @@ static GemmPlan plan_for(int N, int K) {
   } else if (N >= 16384) {
     p.nsub = 4; p.ks = 2;
   } else if (N >= 6144) {
-    p.nsub = 2; p.ks = 8;
+    // K = 8192: four tiles share one pass over X, 160 workgroups for the 10240 columns of the 70B q/k/v
+    // where two tiles make 320, i.e. two on some of the 256 CUs (41.9 us at 25 rows against 32.7)
+    p.nsub = K == 8192 && N > 8192 ? 4 : 2; p.ks = 8;
   } else {
     p.nsub = 1; p.ks = 8;
   }
@@ -803,6 +817,13 @@ static GemmPlan plan_for(int N, int K) {
 // Wide plain-store GEMMs (N >= 65536: vocabulary heads) use gemm_wide_kernel on the same 8-tile
 // packing (a function of the shape only).
 static bool use_wide(const GemmPlan& p) { return p.nsub == 8; }
+
+// Narrow projections whose K is a whole number of 512-wide rounds take X through LDS.
+static bool staged_plan(const GemmPlan& p, int kbt) {
+  if (p.ks != 8) return false;
+  if (kbt == 256) return p.nsub == 2 || p.nsub == 4;
+  return (kbt == 64 || kbt == 128) && p.nsub <= 2;
+}
 
 template <int EPI>
 static int launch_wide(GemmArgs a, int n_groups, hipStream_t s, const WideTopk* tk = nullptr) {
@@ -867,16 +888,18 @@ static int launch_gemm(GemmArgs a, hipStream_t s) {
     }
     const int ct = (b.M + 15) / 16;
     dim3 grid(p.tiles);
-    if (b.kb_total == XS_ROUNDS * 16 && p.ks == 8 && p.nsub <= 2 && ct <= 2) {
-      // K = 4096 narrow projections: x staged through LDS
-#define SSD_GEMM_XS(CT_, NS_)                                                                             \
-  if (ct == CT_ && p.nsub == NS_) {                                                                       \
-    if (b.norm_eps > 0.f)                                                                                 \
-      SSD_LAUNCH((gemm_kernel<CT_, NS_, 8, (CT_ == 1 ? 4 : 2), EPI, 1, true>), grid, dim3(512), 0, s, b); \
-    else                                                                                                  \
-      SSD_LAUNCH((gemm_kernel<CT_, NS_, 8, (CT_ == 1 ? 4 : 2), EPI, 0, true>), grid, dim3(512), 0, s, b); \
+    if (staged_plan(p, b.kb_total)) {  // x staged through LDS
+#define SSD_GEMM_XS(CT_, NS_, XR_)                                                                             \
+  if (ct == CT_ && p.nsub == NS_ && b.kb_total == XR_ * 16) {                                                  \
+    if (b.norm_eps > 0.f)                                                                                      \
+      SSD_LAUNCH((gemm_kernel<CT_, NS_, 8, (CT_ == 1 ? 4 : 2), EPI, 1, XR_>), grid, dim3(512), 0, s, b);       \
+    else                                                                                                       \
+      SSD_LAUNCH((gemm_kernel<CT_, NS_, 8, (CT_ == 1 ? 4 : 2), EPI, 0, XR_>), grid, dim3(512), 0, s, b);       \
   }
-      SSD_GEMM_XS(1, 1) SSD_GEMM_XS(1, 2) SSD_GEMM_XS(2, 1) SSD_GEMM_XS(2, 2)
+#define SSD_GEMM_XSC(NS_, XR_) \
+  SSD_GEMM_XS(1, NS_, XR_) SSD_GEMM_XS(2, NS_, XR_) SSD_GEMM_XS(3, NS_, XR_) SSD_GEMM_XS(4, NS_, XR_)
+      SSD_GEMM_XSC(1, 4) SSD_GEMM_XSC(2, 4) SSD_GEMM_XSC(1, 8) SSD_GEMM_XSC(2, 8) SSD_GEMM_XSC(2, 16) SSD_GEMM_XSC(4, 16)
+#undef SSD_GEMM_XSC
 #undef SSD_GEMM_XS
       int rc = check_launch("gemm");
       if (rc) return rc;
@@ -1132,7 +1155,9 @@ SSD_API int ssd_qkv_rope_finalize_bf16(const float* P, int64_t ldp, int64_t spli
 // (o_proj, bridge out_proj) is fastest as one direct GEMM with the residual add in its epilogue;
 // a long-K projection (down_proj, K = intermediate) as split-K partials plus a finalize that only
 // adds (the direct GEMM would re-read the long activation rows in every workgroup).
-static bool residual_split(int N, int K) { return K > 4096; }
+// Long K is split over workgroups (partials, then a finalize). K = 8192 with N in [6144, 8192] has up to one
+// staged two-tile workgroup per CU instead: 70B o at 25 rows 30.5 us split, 23.2 in one launch.
+static bool residual_split(int N, int K) { return K > 4096 && !(K == 8192 && N >= 6144 && N <= 8192); }
 
 SSD_API int ssd_gemm_residual_group(int N, int K) {
   if (N <= 0 || K <= 0 || K % 32) {
