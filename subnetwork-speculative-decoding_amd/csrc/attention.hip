@@ -21,13 +21,17 @@
 //
 // Kernel structure: attn_partial computes one (m, l, O) partial per (row, superblock) into a
 // workspace -- superblocks below min(P) by workgroups that serve every row at once, the rest by
-// one workgroup per token -- and attn_combine folds the superblocks of each row. S^T = K Q^T and
+// one workgroup per token -- and attn_combine folds the superblocks of each row; contexts of a few
+// superblocks take attn_short, which does both in one launch. S^T = K Q^T and
 // O^T = V^T P^T both run on v_mfma_f32_16x16x32_bf16; the key order inside a block is permuted so
 // the score accumulators are already the P^T operand (no LDS transpose). Row max/sum use
 // cross-lane shuffles of the wave64.
 #include "common.h"
 
 #include <math.h>
+
+#include <algorithm>
+#include <type_traits>
 
 namespace ssd {
 
@@ -137,8 +141,10 @@ __device__ __forceinline__ void load_virtual_frags(Frags<HD>& f, const AttnArgs&
 }
 
 // Patch the ancestor positions of this block into the V^T operands from the ancestors' V^T
-// columns staged in LDS (avt[a][d], a < D): wave-uniform loop over the ancestors in the block.
-template <int HD>
+// columns staged in LDS (avt[a][d], a < D): wave-uniform loop over the ancestors in the block. WHERE
+// names the calling kernel: with a caller of its own the function is specialised for that kernel's LDS
+// addresses before it is inlined (reads with immediate offsets; ~0.2 us of a 13 us call).
+template <int HD, int WHERE = 0>
 __device__ __forceinline__ void patch_ancestors(Frags<HD>& f, const bf16_t (*avt)[HD], int key0, int P, int L,
                                                 int lane) {
   const int i = lane & 15, g = lane >> 4;
@@ -255,6 +261,40 @@ struct alignas(16) AttnLds {
   float l[2][ATT_SB][16];
   bf16_t avt[ATT_MAXD][HD];  // tail: the token's ancestors' V^T columns
 };
+
+// Row rr's four block partials folded in block order: superblock max first, then the weighted sums. A block
+// without keys gets weight 0: its l and O in LDS are finite zeros (published by every wave), and adding an
+// exact zero leaves a sum that is never -0 unchanged, so this equals skipping the block.
+template <int HD>
+struct Folded {
+  float m, l, o[HD / 16];
+};
+template <int HD, typename Lds>
+__device__ __forceinline__ Folded<HD> fold_blocks(const Lds& lds, int area, int rr, int dc) {
+  constexpr int DPT = HD / 16;
+  float mb[ATT_SB], mS = -INFINITY;
+#pragma unroll
+  for (int ww = 0; ww < ATT_SB; ++ww) {
+    mb[ww] = lds.m[area][ww][rr];
+    mS = fmaxf(mS, mb[ww]);
+  }
+  float lS = 0.f, oS[DPT];
+#pragma unroll
+  for (int d = 0; d < DPT; ++d) oS[d] = 0.f;
+#pragma unroll
+  for (int ww = 0; ww < ATT_SB; ++ww) {
+    const float wgt = mb[ww] != -INFINITY ? fast_exp2(mb[ww] - mS) : 0.f;
+    lS = fmaf(lds.l[area][ww][rr], wgt, lS);
+#pragma unroll
+    for (int d = 0; d < DPT; ++d) oS[d] = fmaf(lds.o[area][ww][rr][dc * DPT + d], wgt, oS[d]);
+  }
+  Folded<HD> r;
+  r.m = mS;
+  r.l = lS;
+#pragma unroll
+  for (int d = 0; d < DPT; ++d) r.o[d] = oS[d];
+  return r;
+}
 
 // One launch holds two kinds of workgroups (4 waves; wave w owns block 4*sb + w):
 //  * tail:   (superblock at or beyond min(P), kv head, one token), dispatched first. The wave
@@ -413,41 +453,23 @@ __global__ __launch_bounds__(256, 2) void attn_partial_kernel(AttnArgs a) {
     const int rr = min((int)threadIdx.x >> 4, nv - 1);  // tile row
     const int dc = threadIdx.x & 15;                    // d chunk
     constexpr int DPT = HD / 16;                        // d per thread
-    float mb[ATT_SB], mS = -INFINITY;
-#pragma unroll
-    for (int ww = 0; ww < ATT_SB; ++ww) {
-      mb[ww] = lds.m[buf][ww][rr];
-      mS = fmaxf(mS, mb[ww]);
-    }
-    float lS = 0.f, oS[DPT];
-#pragma unroll
-    for (int d = 0; d < DPT; ++d) oS[d] = 0.f;
-    // A block without keys gets weight 0: its l and O in LDS are finite zeros (published by every
-    // wave), and adding an exact zero leaves a sum that is never -0 unchanged, so this equals
-    // skipping the block.
-#pragma unroll
-    for (int ww = 0; ww < ATT_SB; ++ww) {
-      const float wgt = mb[ww] != -INFINITY ? fast_exp2(mb[ww] - mS) : 0.f;
-      lS = fmaf(lds.l[buf][ww][rr], wgt, lS);
-#pragma unroll
-      for (int d = 0; d < DPT; ++d) oS[d] = fmaf(lds.o[buf][ww][rr][dc * DPT + d], wgt, oS[d]);
-    }
+    const Folded<HD> fr = fold_blocks<HD>(lds, buf, rr, dc);
     const size_t rec = ((size_t)kvh * n_rows + t0 + rr) * a.n_sb_cap + sb;
     // the superblock's normalised output O / l in fp16 (|O / l| <= max |v|; 0 without keys)
-    const float inv = lS > 0.f ? 1.f / lS : 0.f;
+    const float inv = fr.l > 0.f ? 1.f / fr.l : 0.f;
     _Float16* dst = ws_o + rec * HD + dc * DPT;
     if constexpr (DPT % 4 == 0) {
 #pragma unroll
       for (int d = 0; d < DPT; d += 4) {
-        const h16x4_t q = {(_Float16)(oS[d] * inv), (_Float16)(oS[d + 1] * inv), (_Float16)(oS[d + 2] * inv),
-                           (_Float16)(oS[d + 3] * inv)};
+        const h16x4_t q = {(_Float16)(fr.o[d] * inv), (_Float16)(fr.o[d + 1] * inv), (_Float16)(fr.o[d + 2] * inv),
+                           (_Float16)(fr.o[d + 3] * inv)};
         *(h16x4_t*)(dst + d) = q;
       }
     } else {
 #pragma unroll
-      for (int d = 0; d < DPT; ++d) dst[d] = (_Float16)(oS[d] * inv);
+      for (int d = 0; d < DPT; ++d) dst[d] = (_Float16)(fr.o[d] * inv);
     }
-    ws_ml[rec] = make_float2(mS, lS);  // the same pair from each of the row's 16 threads
+    ws_ml[rec] = make_float2(fr.m, fr.l);  // the same pair from each of the row's 16 threads
   };
   u32x4_t qa[KS];
   float m, l;
@@ -584,12 +606,151 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
   }
 }
 
+// Weight of superblock record (m, l) against the row maximum, rounded before it is added (as in the combine).
+__device__ __forceinline__ float record_weight(float m, float l, float mx) {
+#pragma clang fp contract(off)
+  return m == -INFINITY ? 0.f : l * fast_exp2(m - mx);
+}
+
+// Short contexts, in one launch: a workgroup per (token, kv head) of TEAMS teams of 4 waves, team s doing what a
+// tail workgroup of attn_partial does for superblock s; the records meet in LDS instead of the workspace,
+// and the token's rows are combined from there. Same blocks, records and fold, so the same bits as the two
+// launches, of which the second alone is a launch's latency. What is left is that chain once: prefix / ancestors ->
+// K / V -> block -> fold -> combine. Each token reads its own K / V (from L2: a few MB).
+// us per call, two launches / one, 8 kv heads: head_dim 64 -- 1 row of 250 keys 8.8 / 4.7, of 450 8.8 / 5.5, of 1000
+// 9.4 / 8.5, 25 rows of 250 11.0 / 6.8, 64 rows of 250 13.0 / 8.0; head_dim 128 -- 1 row of 250 9.6 / 6.2, of 450
+// 9.5 / 7.8, 25 rows of 250 12.8 / 10.3.
+template <int HD, int TEAMS>
+struct AttnShortLds {
+  float o[TEAMS][ATT_SB][16][HD + 4];
+  float m[TEAMS][ATT_SB][16], l[TEAMS][ATT_SB][16];
+  bf16_t avt[ATT_MAXD][HD];
+  _Float16 rec_o[TEAMS][16][HD + 8];
+  float2 rec_ml[TEAMS][16];
+  int anc[ATT_MAXD];
+};
+
+template <int HD, int TEAMS>
+__global__ __launch_bounds__(256 * TEAMS) void attn_short_kernel(AttnArgs a, bf16_t* __restrict__ out, int64_t ldo) {
+  constexpr int KS = HD / 32, DT = HD / 16, PER = (HD + 63) / 64;
+  __shared__ AttnShortLds<HD, TEAMS> lds;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, team = wave >> 2, w = wave & 3;
+  const int tid = threadIdx.x & 255;
+  const int j = lane & 15, g = lane >> 4;
+  const int rep = a.heads / a.kv_heads;
+  const int kvh = blockIdx.x % a.kv_heads, tok = blockIdx.x / a.kv_heads;
+  const int key0 = (team * ATT_SB + w) * ATT_BLK;
+  const int64_t off = a.kv_off ? a.kv_off[tok] : 0;
+  const bf16_t *Kt = a.K + off, *Vtt = a.Vt + off;
+  const int P = a.prefix[tok], L = P + min(max(a.depth[tok], 0), ATT_MAXD);
+  if (threadIdx.x < ATT_MAXD) lds.anc[threadIdx.x] = a.anc[(size_t)tok * ATT_MAXD + threadIdx.x];
+  __syncthreads();
+  // the ancestors' V^T columns
+  for (int idx = threadIdx.x; idx < (L - P) * HD; idx += 256 * TEAMS) {
+    const int an = idx / HD, d = idx % HD, slot = lds.anc[an];
+    const bool ok = slot >= 0 && slot < a.max_len;
+    const bf16_t h = Vtt[(size_t)kvh * HD * a.max_len + v_off(ok ? slot : 0, d, HD)];
+    lds.avt[an][d] = ok ? h : (bf16_t)0;
+  }
+  Frags<HD> f;
+  uint32_t bits = 0;
+  const bool have = key0 < L && team * ATT_SB * ATT_BLK < a.l_max;
+  if (have) {
+    load_virtual_frags<HD>(f, a, Kt, Vtt, kvh, key0, P, L, lds.anc, lane);
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (logical_slot(key0 + perm_key(kt, 4 * g + e), P, L, lds.anc, a.max_len) >= 0) bits |= 1u << (kt * 4 + e);
+  }
+  if (L > P) {  // uniform
+    __syncthreads();
+    if (have) patch_ancestors<HD, TEAMS>(f, lds.avt, key0, P, L, lane);
+  }
+  for (int t0 = 0; t0 < rep; t0 += 16) {  // one 16-row tile of the token's q heads at every supported shape
+    const int nv = min(16, rep - t0);
+    u32x4_t qf[KS];
+    const bf16_t* qp = a.Q + (size_t)tok * a.ldq + (size_t)(kvh * rep + t0 + min(j, nv - 1)) * HD + g * 8;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *(const u32x4_t*)(qp + ks * 32);
+    float m = -INFINITY, l = 0.f;
+    f32x4_t o[DT];
+    if (have) {
+      block_attend<HD, true>(f, qf, bits, a.scale_log2, m, l, o);
+    } else {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    lds.m[team][w][j] = m;
+    lds.l[team][w][j] = l;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) *(f32x4_t*)&lds.o[team][w][j][dt * 16 + 4 * g] = o[dt];
+    __syncthreads();
+    {  // the team's superblock record: row tid / 16, DPT dims from tid % 16
+      constexpr int DPT = HD / 16;
+      const int rr = tid >> 4, dc = tid & 15;
+      const Folded<HD> fr = fold_blocks<HD>(lds, team, rr, dc);
+      const float inv = fr.l > 0.f ? 1.f / fr.l : 0.f;
+#pragma unroll
+      for (int d = 0; d < DPT; ++d) lds.rec_o[team][rr][dc * DPT + d] = (_Float16)(fr.o[d] * inv);
+      if (dc == 0) lds.rec_ml[team][rr] = make_float2(fr.m, fr.l);
+    }
+    __syncthreads();
+    // combine, one wave per row; lane l owns dims l and l + 64
+    for (int r = wave; r < nv; r += 4 * TEAMS) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int s = 0; s < TEAMS; ++s) mx = fmaxf(mx, lds.rec_ml[s][r].x);
+      float ls = 0.f, os[PER];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) os[i] = 0.f;
+#pragma unroll
+      for (int s = 0; s < TEAMS; ++s) {
+        const float2 ml = lds.rec_ml[s][r];
+        float v[PER];
+#pragma unroll
+        for (int i = 0; i < PER; ++i) v[i] = (float)lds.rec_o[s][r][min(lane + 64 * i, HD - 1)];
+        const float wq = record_weight(ml.x, ml.y, mx);
+        if (wq != 0.f) {
+          ls += wq;
+#pragma unroll
+          for (int i = 0; i < PER; ++i) os[i] = fmaf(v[i], wq, os[i]);
+        }
+      }
+      bf16_t* dst = out + (size_t)tok * ldo + (size_t)(kvh * rep + t0 + r) * HD;
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        if (lane + 64 * i < HD) dst[lane + 64 * i] = f2bf(ls > 0.f ? os[i] / ls : 0.f);
+    }
+    __syncthreads();  // the next tile overwrites the block partials and records
+  }
+}
+
 template <int HD>
 static int launch_attn(AttnArgs a, bf16_t* out, int64_t ldo, hipStream_t s) {
   constexpr int SBK = ATT_BLK * ATT_SB;
   const int n_sb = (a.l_max + SBK - 1) / SBK;
   if (n_sb > a.n_sb_cap) return set_error(SSD_ERANGE, "attention: length %d needs %d superblocks > workspace %d",
                                           a.l_max, n_sb, a.n_sb_cap);
+  auto launch_short = [&](auto teams) {
+    constexpr int TEAMS = decltype(teams)::value;
+    SSD_LAUNCH((attn_short_kernel<HD, TEAMS>), dim3(a.M * a.kv_heads), dim3(256 * TEAMS), 0, s, a, out, ldo);
+    return check_launch("attn_short");
+  };
+  // Whether every workgroup of the launch is resident at once (160 KB of LDS, 2048 threads per CU): a second round
+  // costs what the second launch does (40 rows of 450 keys, head_dim 128: 19.6 us against 15.7 for two
+  // launches; of 900 keys, head_dim 64: 17.4 against 11.8). One superblock's workgroups are those of the two
+  // launches' first, so they win at any number.
+  auto resident = [&](auto teams) {
+    constexpr int TEAMS = decltype(teams)::value;
+    return a.M * a.kv_heads <= 256 * std::min(163840 / (int)sizeof(AttnShortLds<HD, TEAMS>), 8 / TEAMS);
+  };
+  using std::integral_constant;
+  if (n_sb == 1) return launch_short(integral_constant<int, 1>());
+  if (n_sb == 2 && resident(integral_constant<int, 2>())) return launch_short(integral_constant<int, 2>());
+  if constexpr (HD < 128)  // 16 waves of a workgroup leave 128 registers each: not enough for head_dim 128
+    if (n_sb >= 2 && n_sb <= 4 && resident(integral_constant<int, 4>()))
+      return launch_short(integral_constant<int, 4>());
   // rows of several sequences share no keys: every superblock is built per token
   a.n_full = a.kv_off ? 0 : (a.p_min / SBK < n_sb ? a.p_min / SBK : n_sb);
   a.n_tail_sb = n_sb - a.n_full;
@@ -597,13 +758,23 @@ static int launch_attn(AttnArgs a, bf16_t* out, int64_t ldo, hipStream_t s) {
   const uint32_t rep = (uint32_t)(a.heads / a.kv_heads);
   a.rep_magic = (uint32_t)((((uint64_t)1 << 32) + rep - 1) / rep);
   // Shared workgroups split their rows into tile groups when the chip has room for more
-  // workgroups (about 2 per CU resident at once); the groups of one superblock share an XCD.
+  // workgroups (about 2 per CU resident at once); the groups of one superblock share an XCD. The tail's
+  // workgroups (one tile each) count against that room unless a shared workgroup would then go through more
+  // than 9 tiles: by that time the tail's are gone. Microseconds at 64 rows, head_dim 128, 8 q heads per
+  // kv head, counted / not counted: 900 keys 52 / 23, 4000 keys 60 / 38, 8000 keys 72 / 51; with 25 rows and
+  // 4 q heads (7 tiles or fewer in turn), 4000 keys 16.8 / 17.3, 8000 keys 22.6 / 24.4.
   const int units8 = (a.n_full * a.kv_heads + 7) / 8 * 8;
   const int n_tiles = (a.M * (a.heads / a.kv_heads) + 15) / 16;
-  int groups = units8 ? (512 - a.tail_slots) / units8 : 1;
-  groups = groups < 1 ? 1 : (groups > n_tiles ? n_tiles : groups);
-  a.tiles_per_group = (n_tiles + groups - 1) / groups;
-  a.groups = (n_tiles + a.tiles_per_group - 1) / a.tiles_per_group;
+  a.groups = a.tiles_per_group = 1;
+  if (units8) {
+    auto split = [&](int room) {
+      const int groups = std::min(std::max(room / units8, 1), n_tiles);
+      a.tiles_per_group = (n_tiles + groups - 1) / groups;
+    };
+    split(512 - a.tail_slots);
+    if (a.tiles_per_group > 9) split(512);
+    a.groups = (n_tiles + a.tiles_per_group - 1) / a.tiles_per_group;
+  }
   const int grid = a.tail_slots + units8 * a.groups;
   if (grid > 0) {
     SSD_LAUNCH((attn_partial_kernel<HD>), dim3(grid), dim3(256), 0, s, a);
