@@ -864,18 +864,24 @@ __global__ __launch_bounds__(256) void prefill_rowscale_kernel(const bf16_t* __r
 // The tile shapes, largest first, and what a call with each costs: fixed + K / 64 * per-64-k cost *
 // tiles of the busiest CU (two tiles share a CU's time where two workgroups fit). The costs are a
 // least-squares fit (relative error) to the times of q/k/v, o, gate/up and down of the 1B, 8B and 70B shapes
-// at 23 M from 24 to 4096 with every shape (us, this card); the rule's choice is within 1.2 % of the
-// fastest shape on average there (worst 21 %). Large tiles move the fewest operand bytes per MFMA;
+// at 23 M from 24 to 4096 with every shape (us, this card; the five shapes of 96, 160 and 192 tokens at
+// 24 M, 1B and 8B); the rule's choice is within 1.2 % of the fastest shape on average. Large tiles move the fewest operand bytes per MFMA;
 // small ones put a short prompt's few rows on all CUs (M = 512, N = 4096, K = 14336: 32 tiles of 256
 // x 256 279 us, 256 of 128 x 64 90 us).
+// The shapes of 96, 160 and 192 tokens are for the row counts that 64, 128 and 256 pad the most: gate/up
+// at N = 28672, K = 4096 -- 160 rows 71 us on 128-token tiles, 54 on 160; 350 rows 110 on 256, 84 on 192;
+// down at 1150 rows 176 on 128, 134 on 160. Over 200 calls of the 1B and 8B shapes at 24 M from 66 to 4096
+// the choice among all is 3.8 % faster (geometric mean) than among the other nine, at worst 2 % slower.
 struct PrefillTile {
   int xt, yt, occ;
   double fixed, one, two;  // us; per 64 k with one tile on a CU, with two side by side (occ 2)
 };
 constexpr PrefillTile PREFILL_TILES[] = {
-    {8, 8, 1, 14.2, 1.275, 0}, {6, 8, 1, 10.5, 1.032, 0},     {8, 4, 1, 3.0, 0.876, 0},
-    {6, 4, 1, 1.9, 0.746, 0},  {4, 4, 1, 4.0, 0.509, 0},      {4, 2, 1, 2.9, 0.364, 0},
-    {2, 2, 2, 2.7, 0.233, 0.418}, {1, 2, 2, 3.1, 0.178, 0.294}, {1, 1, 2, 4.2, 0.121, 0.208},
+    {8, 8, 1, 14.2, 1.275, 0}, {6, 8, 1, 10.5, 1.032, 0},         {8, 6, 1, 11.3, 1.03, 0},
+    {8, 4, 1, 3.0, 0.876, 0},  {6, 4, 1, 1.9, 0.746, 0},          {4, 6, 1, 7.8, 0.701, 0},
+    {4, 5, 1, 4.0, 0.627, 0},  {4, 4, 1, 4.0, 0.509, 0},          {4, 3, 1, 6.3, 0.424, 0},
+    {4, 2, 1, 2.9, 0.364, 0},  {2, 3, 2, 3.5, 0.299, 0.509},      {2, 2, 2, 2.7, 0.233, 0.418},
+    {1, 2, 2, 3.1, 0.178, 0.294}, {1, 1, 2, 4.2, 0.121, 0.208},
 };
 constexpr int N_PREFILL_TILES = sizeof(PREFILL_TILES) / sizeof(PREFILL_TILES[0]);
 
@@ -919,12 +925,17 @@ static int launch_prefill_gemm4(const GemmArgs& a, int group, int pos0, int cus,
     case 0:
       if constexpr (EPI != EPI_QKV) return launch_prefill_tile<EPI, 8, 8, 1, 4, 1>(a, group, pos0, cus, s);
     case 1: return launch_prefill_tile<EPI, 6, 8, 1, 4, 1>(a, group, pos0, cus, s);
-    case 2: return launch_prefill_tile<EPI, 8, 4, 1, 4, 1>(a, group, pos0, cus, s);
-    case 3: return launch_prefill_tile<EPI, 6, 4, 1, 4, 1>(a, group, pos0, cus, s);
-    case 4: return launch_prefill_tile<EPI, 4, 4, 2, 5, 1>(a, group, pos0, cus, s);
-    case 5: return launch_prefill_tile<EPI, 4, 2, 2, 6, 1>(a, group, pos0, cus, s);
-    case 6: return launch_prefill_tile<EPI, 2, 2, 2, 5, 2>(a, group, pos0, cus, s);
-    case 7: return launch_prefill_tile<EPI, 1, 2, 2, 6, 2>(a, group, pos0, cus, s);
+    case 2: return launch_prefill_tile<EPI, 8, 6, 1, 4, 1>(a, group, pos0, cus, s);
+    case 3: return launch_prefill_tile<EPI, 8, 4, 1, 4, 1>(a, group, pos0, cus, s);
+    case 4: return launch_prefill_tile<EPI, 6, 4, 1, 4, 1>(a, group, pos0, cus, s);
+    case 5: return launch_prefill_tile<EPI, 4, 6, 1, 4, 1>(a, group, pos0, cus, s);
+    case 6: return launch_prefill_tile<EPI, 4, 5, 2, 4, 1>(a, group, pos0, cus, s);
+    case 7: return launch_prefill_tile<EPI, 4, 4, 2, 5, 1>(a, group, pos0, cus, s);
+    case 8: return launch_prefill_tile<EPI, 4, 3, 2, 5, 1>(a, group, pos0, cus, s);
+    case 9: return launch_prefill_tile<EPI, 4, 2, 2, 6, 1>(a, group, pos0, cus, s);
+    case 10: return launch_prefill_tile<EPI, 2, 3, 2, 4, 2>(a, group, pos0, cus, s);
+    case 11: return launch_prefill_tile<EPI, 2, 2, 2, 5, 2>(a, group, pos0, cus, s);
+    case 12: return launch_prefill_tile<EPI, 1, 2, 2, 6, 2>(a, group, pos0, cus, s);
     default: return launch_prefill_tile<EPI, 1, 1, 2, 8, 2>(a, group, pos0, cus, s);
   }
 }

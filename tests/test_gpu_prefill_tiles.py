@@ -43,10 +43,11 @@ def _run(epi, x, m, wp, grp, n, k, res, pos0=0, qkv_shape=None):
     return (out, *kv)
 
 
-# N, K and row counts around the tiles' 32 / 64 / 128 / 256 rows; wide N makes the large tiles the cheapest
+# N, K and row counts around the tiles' 32 / 64 / 96 / 128 / 160 / 192 / 256 rows; wide N makes the large tiles the cheapest
 @pytest.mark.parametrize("epi,n,k,qkv_shape", [("store", 4096, 4096, None), ("store", 200, 192, None),
                                                ("store", 28672, 256, None), ("swiglu", 28672, 512, None),
-                                               ("swiglu", 1056, 2048, None), ("qkv", 6144, 4096, (32, 8, 128)),
+                                               ("swiglu", 1056, 2048, None), ("swiglu", 16384, 2048, None),
+                                               ("qkv", 6144, 4096, (32, 8, 128)), ("qkv", 3072, 2048, (32, 8, 64)),
                                                ("qkv", 3072, 64, (32, 8, 64))])
 def test_rows_have_the_same_bits_on_every_tile_shape(epi, n, k, qkv_shape):
     from ssd import ops
@@ -58,7 +59,7 @@ def test_rows_have_the_same_bits_on_every_tile_shape(epi, n, k, qkv_shape):
     wp = ops.pack_weight(w)
     pos0 = 5 if qkv_shape else 0
     ref = _run(epi, x, top, wp, grp, n, k, res, pos0, qkv_shape)
-    for m in (1, 31, 32, 33, 64, 65, 96, 127, 129, 200, 257, 300, 513, 700, 900):
+    for m in (1, 31, 32, 33, 64, 65, 96, 127, 129, 161, 200, 257, 300, 350, 450, 513, 700, 900):
         got = _run(epi, x, m, wp, grp, n, k, res, pos0, qkv_shape)
         assert torch.equal(got[0], ref[0][:m]), (epi, m)
         for a, b in zip(got[1:], ref[1:]):
@@ -71,9 +72,25 @@ def test_rows_have_the_same_bits_on_every_tile_shape(epi, n, k, qkv_shape):
         assert ((ref[0].float() - want).abs() <= 2 ** -7 * p.abs() + 2 ** -8 * want.abs() + 1e-3).all()
 
 
+# the 192-token shapes' plain and q/k/v write-outs, whose cheapest calls are longer ones
+@pytest.mark.parametrize("epi,n,k,qkv_shape", [("store", 4096, 4096, None), ("qkv", 6144, 4096, (32, 8, 128))])
+def test_long_calls_have_the_same_bits_on_every_tile_shape(epi, n, k, qkv_shape):
+    from ssd import ops
+
+    x, w = _rand(3000, k, seed=12), _rand(n, k, seed=13, std=0.02)
+    res, grp, wp = _rand(3000, n, seed=14), ops.weight_group(n, k), ops.pack_weight(w)
+    ref = _run(epi, x, 3000, wp, grp, n, k, res, 3, qkv_shape)
+    for m in (1150, 1300, 1500, 1800, 2500):
+        got = _run(epi, x, m, wp, grp, n, k, res, 3, qkv_shape)
+        assert torch.equal(got[0], ref[0][:m]), (epi, m)
+        for a, b in zip(got[1:], ref[1:]):
+            assert torch.equal(a, b[:, :m]), (epi, m)
+
+
 # k loops shorter than, equal to and just past the operand ring's depth (K / 64 = 1 .. 9), on the
-# smallest tile (N = 64) and on the largest (N = 28672, M = 4096: the cheapest from K = 192 on)
-@pytest.mark.parametrize("m,n,k", [(m, n, k) for m, n in ((40, 64), (700, 640)) for k in range(64, 577, 64)]
+# smallest tile (N = 64), tiles between, and on the largest (N = 28672, M = 4096: the cheapest from K = 192 on)
+@pytest.mark.parametrize("m,n,k", [(m, n, k) for m, n in ((40, 64), (700, 640), (290, 16384), (190, 16384))
+                                   for k in range(64, 577, 64)]
                          + [(4096, 28672, k) for k in (192, 256, 320)])
 def test_short_k_loops_match_the_fp32_product(m, n, k):
     from ssd import ops
