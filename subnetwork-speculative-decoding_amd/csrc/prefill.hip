@@ -171,12 +171,18 @@ __device__ __forceinline__ void p4_step(const char* const (&wp)[LW], const char*
   }
 }
 
-// SiLU of the prefill's SwiGLU staging: x sigma(x) with the logistic function through the hardware
-// base-2 exponential and reciprocal, 1 / (1 + 2^(-x log2 e)) (a few ulp of fp32, then rounded to
-// bf16; the exact division and exponential of silu_f cost half of the gate/up tile's staging).
-// exp2 overflows to +inf for x < -88 (sigma = 0, silu = -0) and underflows to 0 for large x (silu = x).
+// SiLU of the prefill's SwiGLU staging: x / (1 + 2^(-x log2 e)) through the hardware base-2 exponential and
+// reciprocal, the quotient corrected by its residual. Both sides of the quotient carry a factor of 1/16, which
+// keeps the reciprocal normal where the exponential is near 2^128 (exact for a bf16 x, subnormal ones too); the
+// fixup gives the quotients by infinity (x < -88.7: -0; x = -inf: NaN). x is a rounded bf16 value and the result is
+// rounded to bf16, so the whole range is 65280 finite inputs: every one gives silu_f's bf16 value, i.e. that of
+// the decode kernels. Without the correction 5.9375 and -87.5 .. -88.5 did not (the last flushed to -0). The
+// four instructions more cost nothing that is measured; silu_f's own division and exponential cost half of
+// the gate/up tile's staging.
 __device__ __forceinline__ float pf_silu(float x) {
-  return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
+  const float d = fmaf(__builtin_amdgcn_exp2f(x * -1.4426950408889634f), 0.0625f, 0.0625f), n = x * 0.0625f;
+  const float r = __builtin_amdgcn_rcpf(d), q = n * r;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, n), r, q), d, n);
 }
 
 // q/k/v write-out of one staged tile: rows of q and K-cache slots (RoPE applied here), then 8-slot
