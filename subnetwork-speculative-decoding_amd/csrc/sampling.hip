@@ -1121,7 +1121,8 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_walk_kernel(AcceptArgs a, 
   __shared__ StateScalars st_sh[16];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int C = a.ws.C, n_rows = min(verify_nodes(a.tree) + 1, a.rows);
-  if (threadIdx.x < n_rows - 1) tok_sh[threadIdx.x] = a.tree.vtokens[threadIdx.x];
+  // every node's token: a row's accepted child may lie beyond the launch's rows
+  if (threadIdx.x < verify_nodes(a.tree)) tok_sh[threadIdx.x] = a.tree.vtokens[threadIdx.x];
   NodeKids& kids = kids_sh[wv];  // this wave's own, read back by the lanes that wrote them or in step with them
   StateScalars& s = st_sh[wv];
   for (int r = wv; r < n_rows; r += 16) {

@@ -310,6 +310,20 @@ def test_accept_sample_leaf_root_and_empty_tree():
     assert acc == [] and (frag or bonus == want)
 
 
+@pytest.mark.parametrize("rows", [1, 2, 3])
+def test_accept_sample_of_a_tree_larger_than_its_rows(rows):
+    """Rows for the root and the first rows - 1 of three children: the third, the only token the target
+    allows, is accepted with its own token, and the walk ends there without a draw (bonus 0)."""
+    V = 50
+    P = torch.zeros(rows, V)
+    P[:, 21] = 1
+    q = torch.zeros(V)
+    q[[7, 9, 21]] = 1 / 3
+    t = device_tree([7, 9, 21], [-1, -1, -1], [0, 1, 2])
+    for ctr in range(4):
+        assert accept_on_gpu(t, P, {-1: q}, V, 5, ctr, max_kids=3) == ([2], 0)
+
+
 @pytest.mark.parametrize("top_p", [1.0, 0.9])
 def test_first_committed_token_is_target_distributed(top_p):
     """The isolated-acceptance check at the 8B vocabulary: target logits N(0, 4^2), draft =
