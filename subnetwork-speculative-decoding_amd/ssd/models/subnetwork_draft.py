@@ -575,11 +575,16 @@ class SubnetworkDraftModel(nn.Module):
                         past_key_values: Optional[KVCache]) -> DraftOutput:
         """forward() of a long causal prompt: the MFMA prefill kernels, PREFILL_CHUNK rows per call, one
         final-norm launch per chunk, and the head on the rows asked for."""
+        if ids.dim() != 1:
+            raise ValueError(f"input_ids must be [1, tokens], got {ids.dim() + 1} dimensions")
         q, past = ids.numel(), cache.get_seq_length()
         ids = ids.cpu()
-        host = ids.to(torch.int32)
-        if ids.dtype == torch.int64 and not torch.equal(host.to(torch.int64), ids):
-            raise RuntimeError("token ids cannot be converted to int32 without overflow")
+        if ids.dtype == torch.int64:
+            host = ids.to(torch.int32)
+            if not torch.equal(host.to(torch.int64), ids):
+                raise RuntimeError("token ids cannot be converted to int32 without overflow")
+        else:  # by value: what an int32 cannot hold is refused
+            host = ids if ids.dtype == torch.int32 else torch.tensor(ids.tolist(), dtype=torch.int32)
         ws = self.workspace(CHUNK)
         n_keep = 0 if not compute_logits else min(logits_to_keep, q) if logits_to_keep > 0 else q
         hidden = torch.empty(q, self.d_model, dtype=torch.bfloat16, device=self.model.device)

@@ -27,3 +27,33 @@ def test_forward_returns_the_rows_asked_for(monkeypatch, tokens, chunk):
     assert target(ids, past_key_values=target.new_cache(tokens), compute_logits=False).logits is None
     with pytest.raises(RuntimeError):
         target(torch.full((1, tokens), 1 << 40), past_key_values=target.new_cache(tokens))
+
+
+@pytest.fixture(scope="module")
+def target():
+    from ssd.engine.speculative import TargetRunner
+    from ssd.models.llama import LlamaShape, MI355XLlama
+
+    return TargetRunner(MI355XLlama.synthetic(LlamaShape(256, 2, 4, 2, 64, 512, 1000), seed=3))
+
+
+@pytest.mark.parametrize("bad", [torch.zeros(1, 65, 2, dtype=torch.int64), torch.zeros(1, 65, 1, dtype=torch.int64),
+                                 torch.full((1, 65), 4_000_000_000, dtype=torch.uint32),
+                                 torch.full((1, 65), 1 << 40, dtype=torch.uint64), torch.full((1, 65), 3e9),
+                                 torch.full((1, 65), float("nan"))], ids=lambda t: f"{tuple(t.shape)}-{t.dtype}".replace("torch.", ""))
+def test_long_prompts_refuse_what_short_ones_refuse(target, bad):
+    """Ids that are no [1, tokens] table or do not fit int32, from a prompt that runs on the prefill kernels and
+    from one of 8 tokens on the decode kernels. The cache is left as it was."""
+    for n in (65, 8):
+        cache = target.new_cache(192)
+        with pytest.raises((RuntimeError, ValueError)):
+            target(bad[:, :n], past_key_values=cache)
+        assert cache.get_seq_length() == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int16, torch.uint8, torch.float32])
+def test_long_prompts_take_ids_of_any_type(target, dtype):
+    ids = torch.randint(0, 200, (1, 70), generator=torch.Generator().manual_seed(1))
+    want = target(ids, past_key_values=target.new_cache(80)).logits
+    for x in (ids.to(dtype), ids.to(dtype).cuda()):
+        assert torch.equal(target(x, past_key_values=target.new_cache(80)).logits, want)
