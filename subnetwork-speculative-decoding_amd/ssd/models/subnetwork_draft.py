@@ -356,7 +356,7 @@ class SubnetworkDraftModel(nn.Module):
 
     def prefill_chunk(self, ids, pos0: int, cache: KVCache, logits: bool) -> Optional[torch.Tensor]:
         """ssd_prefill over prompt rows pos0 .. pos0 + len(ids) - 1 (at most PREFILL_CHUNK; ``ids`` a list
-        or a host int32 tensor): K/V of every layer into the cache, the final residual stream in the
+        or an int32 tensor): K/V of every layer into the cache, the final residual stream in the
         prefill workspace's h, and with ``logits`` the last row's full-vocabulary logits ([1, V] view)."""
         m = len(ids)
         if m > PREFILL_CHUNK:
@@ -364,9 +364,12 @@ class SubnetworkDraftModel(nn.Module):
         pw = self._pw
         if pw is None or pw.m_cap < m:
             pw = self._pw = PrefillWorkspace(self.model, max(m, min(PREFILL_CHUNK, 1024)))
-        # from pinned memory, so that the layers are enqueued without waiting for the copy (the allocator
-        # keeps the block until the stream has read it)
-        pw.ids[:m].copy_(torch.as_tensor(ids, dtype=torch.int32).pin_memory(), non_blocking=True)
+        src = torch.as_tensor(ids, dtype=torch.int32)
+        if src.device.type == "cpu":
+            # a pinned copy of this call's own, so that the layers are enqueued without waiting for the transfer and
+            # the caller may change ``ids`` at once (the allocator keeps the block until the stream has read it)
+            src = torch.empty(m, dtype=torch.int32, pin_memory=True).copy_(src)
+        pw.ids[:m].copy_(src, non_blocking=True)
         _lib.call("ssd_prefill", self.model.native(cache.capacity), self.model.lm_head.data_ptr() if logits else None,
                   pw.native(cache), pw.ids.data_ptr(), m, int(pos0), ops.stream())
         return pw.logits if logits else None

@@ -57,3 +57,19 @@ def test_long_prompts_take_ids_of_any_type(target, dtype):
     want = target(ids, past_key_values=target.new_cache(80)).logits
     for x in (ids.to(dtype), ids.to(dtype).cuda()):
         assert torch.equal(target(x, past_key_values=target.new_cache(80)).logits, want)
+
+
+@pytest.mark.parametrize("kind", ["list", "pageable", "pinned", "device"])
+def test_prefill_chunk_has_taken_its_ids_when_it_returns(target, kind):
+    """The transfer of the ids is not waited for, so a caller who reuses a buffer of any kind must not change them. The
+    stream is held busy until after the buffer is overwritten."""
+    ids = torch.randint(0, 1000, (70,), generator=torch.Generator().manual_seed(2), dtype=torch.int32)
+    cache = target.new_cache(128)
+    cache.ensure(target.num_kv_heads, target.head_dim, target.model.device)
+    want = target.prefill_chunk(ids.tolist(), 0, cache, True).clone()
+    buf = {"list": ids.tolist(), "pageable": ids.clone(), "pinned": ids.pin_memory(), "device": ids.cuda()}[kind]
+    torch.cuda.synchronize()
+    torch.cuda._sleep(20_000_000)  # about 10 ms
+    got = target.prefill_chunk(buf, 0, cache, True)
+    buf[:] = [0] * 70 if kind == "list" else torch.zeros(70, dtype=torch.int32)
+    assert torch.equal(got, want)
