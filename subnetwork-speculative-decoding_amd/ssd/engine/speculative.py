@@ -42,7 +42,7 @@ from ssd.config import DraftingConfig
 from ssd.engine.kv_cache import KVCache
 from ssd.engine.sampling import Sampler
 from ssd.engine.tree_drafter import TREE_CAP, DeviceTree, TreeDrafter
-from ssd.models.subnetwork_draft import CHUNK, PREFILL_CHUNK, PREFILL_MIN, Rows, SubnetworkDraftModel
+from ssd.models.subnetwork_draft import CHUNK, PREFILL_CHUNK, Rows, SubnetworkDraftModel, prefill_kernels_win
 
 
 @dataclass
@@ -100,16 +100,16 @@ class _Phases:
 
 def _prefill_logits(target: SubnetworkDraftModel, ids: list, cache: KVCache, ws) -> torch.Tensor:
     """Target forward over the prompt into ``cache`` (reference speculative.py:149-151); returns the
-    last row's logits (a [1, V] view of a buffer the next forward reuses). Prompts of at least
-    PREFILL_MIN tokens run on the MFMA prefill kernels (chunks of PREFILL_CHUNK rows), shorter
-    ones as causal rows through the decode forward (chunks of 64)."""
+    last row's logits (a [1, V] view of a buffer the next forward reuses). Prompts longer than a decode
+    forward run on the MFMA prefill kernels (chunks of PREFILL_CHUNK rows) unless the cached past is long
+    (prefill_kernels_win), the others as causal rows through the decode forward (chunks of 64)."""
     dev = target.model.device
     past = cache.get_seq_length()
     q = len(ids)
     cache.check_room(past + q)
     cache.ensure(target.num_kv_heads, target.head_dim, dev)
     logits = None
-    if q >= PREFILL_MIN and target.prefill_capable():
+    if prefill_kernels_win(q, past) and target.prefill_capable():
         for c0 in range(0, q, PREFILL_CHUNK):
             c1 = min(q, c0 + PREFILL_CHUNK)
             logits = target.prefill_chunk(ids[c0:c1], past + c0, cache, c1 == q)

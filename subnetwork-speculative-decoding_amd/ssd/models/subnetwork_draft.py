@@ -36,10 +36,16 @@ from ssd.models.llama import MI355XLlama
 
 MAXD = 32        # ancestors per row (ssd_attn_max_depth)
 CHUNK = 64       # rows per kernel launch chain (GEMM column tiles of 16 x 4)
-# Causal prompts at least this long run on the MFMA prefill kernels: everything past one decode forward of
-# CHUNK rows. One 8B layer, us: 64 rows 131 through the decode kernels, 117 through the prefill kernels; 100
-# rows 255 (two decode forwards) against 137; 32 rows 90 against 112.
+# Causal prompts that run on the MFMA prefill kernels: everything past one decode forward of CHUNK rows, except
+# short ones after a long cached past. One 8B layer, us: 64 rows 131 through the decode kernels, 117 through the
+# prefill kernels; 100 rows 255 (two decode forwards) against 137; 32 rows 90 against 112. The prefill attention
+# has one workgroup for 16 or 32 rows of 4 heads walk all their keys, while decode attention spreads the keys
+# over the chip, so a long past turns this round: the two meet at 7900 cached tokens for 65 rows of 24 heads
+# (3B; 15000 at 1B and 8B, 33000 at 70B), 12500 for 128 (24000, 45000), 35000 for 255 (75000 and more). 100 rows after
+# 64000 tokens, 8B: 654 a layer through the decode kernels, 1083 through the prefill kernels.
 PREFILL_MIN = CHUNK + 1
+PREFILL_ANY_PAST = 256  # rows from which the past does not matter (four decode forwards)
+PREFILL_PAST = 96       # below that: cached tokens per row up to which the prefill kernels are the faster
 PREFILL_CHUNK = 4096  # prompt rows per ssd_prefill call
 
 
@@ -88,6 +94,11 @@ def as_device_model(base) -> MI355XLlama:
         cached = MI355XLlama.from_hf(base, dev)
         base._ssd_mi355x = cached
     return cached
+
+
+def prefill_kernels_win(rows: int, past: int) -> bool:
+    """Whether a causal prompt of ``rows`` after ``past`` cached tokens is one for the prefill kernels."""
+    return rows >= PREFILL_ANY_PAST or (rows >= PREFILL_MIN and past <= PREFILL_PAST * rows)
 
 
 class Rows:
@@ -527,7 +538,7 @@ class SubnetworkDraftModel(nn.Module):
         past = cache.get_seq_length()
         cache.check_room(past + q)
         pos = None if position_ids is None else torch.as_tensor(position_ids).reshape(-1).tolist()
-        if (tree_attention_mask is None and not output_bridge_states and q >= PREFILL_MIN and self.prefill_capable()
+        if (tree_attention_mask is None and not output_bridge_states and prefill_kernels_win(q, past) and self.prefill_capable()
                 and (pos is None or pos == list(range(past, past + q)))):
             return self._forward_prompt(ids[0], cache, logits_to_keep, compute_logits, past_key_values)
         ids = ids[0].tolist()

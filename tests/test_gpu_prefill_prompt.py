@@ -73,3 +73,24 @@ def test_prefill_chunk_has_taken_its_ids_when_it_returns(target, kind):
     got = target.prefill_chunk(buf, 0, cache, True)
     buf[:] = [0] * 70 if kind == "list" else torch.zeros(70, dtype=torch.int32)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("tokens,past,decode", [(64, 0, True), (65, 0, False), (65, 6240, False), (65, 6241, True),
+                                                (100, 9600, False), (100, 12000, True), (255, 24480, False),
+                                                (255, 24481, True), (256, 30000, False)])
+def test_short_prompts_after_a_long_past_run_on_the_decode_kernels(target, tokens, past, decode):
+    """Past the line the rows' bits are the decode forward's (an explicit causal mask always takes that one),
+    before it they are not."""
+    ids = torch.randint(0, 1000, (1, tokens), generator=torch.Generator().manual_seed(5))
+    cache = target.new_cache(past + tokens)
+    cache.ensure(target.num_kv_heads, target.head_dim, target.model.device)
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    cache.k.normal_(generator=gen)
+    cache.vt.normal_(generator=gen)
+    out = []
+    for mask in (None, torch.ones(tokens, tokens).tril().bool()[None, None]):
+        cache.reset()
+        cache.advance(past)
+        out.append(target(ids, past_key_values=cache, tree_attention_mask=mask).hidden_states)
+    assert torch.equal(*out) == decode
+    torch.testing.assert_close(out[0].float(), out[1].float(), rtol=0.1, atol=0.1)
