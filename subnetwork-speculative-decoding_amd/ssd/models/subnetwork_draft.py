@@ -374,7 +374,8 @@ class SubnetworkDraftModel(nn.Module):
             raise ValueError(f"prefill chunk of {m} rows > {PREFILL_CHUNK}")
         pw = self._pw
         if pw is None or pw.m_cap < m:
-            pw = self._pw = PrefillWorkspace(self.model, max(m, min(PREFILL_CHUNK, 1024)))
+            # room for 256 rows while prompts are short (27 MB at 70B), then for 1024 (109 MB), then what is asked for
+            pw = self._pw = PrefillWorkspace(self.model, max(m, min(PREFILL_CHUNK, 256 if m <= 256 else 1024)))
         src = torch.as_tensor(ids, dtype=torch.int32)
         if src.device.type == "cpu":
             # a pinned copy of this call's own, so that the layers are enqueued without waiting for the transfer and

@@ -94,3 +94,16 @@ def test_short_prompts_after_a_long_past_run_on_the_decode_kernels(target, token
         out.append(target(ids, past_key_values=cache, tree_attention_mask=mask).hidden_states)
     assert torch.equal(*out) == decode
     torch.testing.assert_close(out[0].float(), out[1].float(), rtol=0.1, atol=0.1)
+
+
+def test_prefill_workspace_follows_the_prompts(target):
+    """A short prompt does not hold the buffers of a long one; they grow, and results stay."""
+    target._pw = None
+    ids = torch.randint(0, 1000, (1, 2000), generator=torch.Generator().manual_seed(7))
+    first, rows = None, []
+    for n in (65, 256, 257, 100, 1024, 2000):
+        out = target(ids[:, :n], past_key_values=target.new_cache(n)).hidden_states
+        rows.append(target._pw.m_cap)
+        first = out if first is None else first
+        assert torch.equal(out[:, :65], first)
+    assert rows == [256, 256, 1024, 1024, 1024, 2000]
