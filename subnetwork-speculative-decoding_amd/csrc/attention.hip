@@ -621,7 +621,7 @@ __device__ __forceinline__ float record_weight(float m, float l, float mx) {
 // 9.4 / 8.5, 25 rows of 250 11.0 / 6.8, 64 rows of 250 13.0 / 8.0; head_dim 128 -- 1 row of 250 9.6 / 6.2, of 450
 // 9.5 / 7.8, 25 rows of 250 12.8 / 10.3.
 template <int HD, int TEAMS>
-struct AttnShortLds {
+struct alignas(16) AttnShortLds {  // o's rows are written 16 bytes at a time
   float o[TEAMS][ATT_SB][16][HD + 4];
   float m[TEAMS][ATT_SB][16], l[TEAMS][ATT_SB][16];
   bf16_t avt[ATT_MAXD][HD];
@@ -634,6 +634,7 @@ template <int HD, int TEAMS>
 __global__ __launch_bounds__(256 * TEAMS) void attn_short_kernel(AttnArgs a, bf16_t* __restrict__ out, int64_t ldo) {
   constexpr int KS = HD / 32, DT = HD / 16, PER = (HD + 63) / 64;
   __shared__ AttnShortLds<HD, TEAMS> lds;
+  static_assert(alignof(AttnShortLds<HD, TEAMS>) >= 16 && sizeof(lds.o[0][0][0]) % 16 == 0, "16-byte stores to lds.o");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, team = wave >> 2, w = wave & 3;
   const int tid = threadIdx.x & 255;
   const int j = lane & 15, g = lane >> 4;
