@@ -738,19 +738,24 @@ static int launch_attn(AttnArgs a, bf16_t* out, int64_t ldo, hipStream_t s) {
     SSD_LAUNCH((attn_short_kernel<HD, TEAMS>), dim3(a.M * a.kv_heads), dim3(256 * TEAMS), 0, s, a, out, ldo);
     return check_launch("attn_short");
   };
-  // Whether every workgroup of the launch is resident at once (160 KB of LDS, 2048 threads per CU): a second round
-  // costs what the second launch does (40 rows of 450 keys, head_dim 128: 19.6 us against 15.7 for two
-  // launches; of 900 keys, head_dim 64: 17.4 against 11.8). One superblock's workgroups are those of the two
-  // launches' first, so they win at any number.
-  auto resident = [&](auto teams) {
+  // How many workgroups the one launch may have: four teams as many as are resident at once, one per CU (their 16
+  // waves' registers fill it at every head_dim, their LDS at 64), since a second round costs more than the
+  // second launch does (us, two launches / one, 900 keys: 40 rows, 8 kv heads, head_dim 64 11.8 / 17.4, head_dim
+  // 32 10.8 / 13.4; 25 rows, 16 kv heads, head_dim 32 10.2 / 13.5). Two teams as many as LDS and threads hold, one
+  // per CU at head_dim 128 (40 rows of 450 keys: 15.7 / 19.6), three at 64 and four at 32: registers hold one
+  // fewer, and the few that wait still cost less than the second launch (16 kv heads, head_dim 64, 260 / 400 /
+  // 505 keys: 33 rows 14.2 / 9.1, 13.8 / 11.2, 14.0 / 11.2; 40 rows 15.7 / 12.1, 13.8 / 13.8, 14.2 / 13.8). One
+  // superblock's workgroups are those of the two launches' first, so they win at any number.
+  auto fits = [&](auto teams) {
     constexpr int TEAMS = decltype(teams)::value;
-    return a.M * a.kv_heads <= 256 * std::min(163840 / (int)sizeof(AttnShortLds<HD, TEAMS>), 8 / TEAMS);
+    constexpr int PER_CU = TEAMS == 4 ? 1 : std::min(163840 / (int)sizeof(AttnShortLds<HD, TEAMS>), 8 / TEAMS);
+    return a.M * a.kv_heads <= 256 * PER_CU;
   };
   using std::integral_constant;
   if (n_sb == 1) return launch_short(integral_constant<int, 1>());
-  if (n_sb == 2 && resident(integral_constant<int, 2>())) return launch_short(integral_constant<int, 2>());
+  if (n_sb == 2 && fits(integral_constant<int, 2>())) return launch_short(integral_constant<int, 2>());
   if constexpr (HD < 128)  // 16 waves of a workgroup leave 128 registers each: not enough for head_dim 128
-    if (n_sb >= 2 && n_sb <= 4 && resident(integral_constant<int, 4>()))
+    if (n_sb >= 2 && n_sb <= 4 && fits(integral_constant<int, 4>()))
       return launch_short(integral_constant<int, 4>());
   // rows of several sequences share no keys: every superblock is built per token
   a.n_full = a.kv_off ? 0 : (a.p_min / SBK < n_sb ? a.p_min / SBK : n_sb);

@@ -30,7 +30,7 @@ def _case(m, heads, kvh, hd, L, seed):
     return q, k, v, prefix, anc
 
 
-def _call(case, rows, p_min, l_max):
+def _call(case, rows, p_min, l_max, ws=None):
     from ssd import ops
 
     q, k, v, prefix, anc = case
@@ -39,7 +39,7 @@ def _call(case, rows, p_min, l_max):
     for i, t in enumerate(rows):
         an[i, :len(anc[t])] = torch.tensor(anc[t], dtype=torch.int32)
     i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
-    ws = torch.zeros(ops.attn_workspace_floats(m, heads, hd, CAP), device=DEV)
+    ws = torch.zeros(ops.attn_workspace_floats(m, heads, hd, CAP), device=DEV) if ws is None else ws
     out = torch.full((m, heads * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
     qd = q[rows].reshape(m, heads * hd).to(DEV)
     ops.tree_attention(qd, m, heads, kvh, hd, ops.kv_tile(k.to(DEV), "k"), ops.kv_tile(v.to(DEV), "v"), CAP,
@@ -77,3 +77,17 @@ def test_tile_groups_leave_the_rows_alone(hd, heads, kvh, m, P):
     got = _call(case, list(range(m)), P, P + 8)
     for t in (0, 1, m // 2, m - 1):
         assert torch.equal(got[t:t + 1], _call(case, [t], P, P + 8)), t
+
+
+# the last row count of each kind that takes one launch; the next takes two
+@pytest.mark.parametrize("hd,heads,kvh,L,last", [(32, 32, 8, 1024, 32), (32, 32, 16, 600, 16), (32, 32, 16, 512, 64),
+                                                 (64, 32, 8, 1024, 32), (64, 32, 16, 512, 48), (64, 32, 8, 512, 96),
+                                                 (128, 32, 8, 512, 32)])
+def test_one_launch_only_while_its_workgroups_fit(hd, heads, kvh, L, last):
+    """One launch keeps its records in LDS, two pass them through the workspace."""
+    from ssd import ops
+
+    for m in (last, last + 1):
+        ws = torch.full((ops.attn_workspace_floats(m, heads, hd, CAP),), -7.0, device=DEV)
+        _call(_case(m, heads, kvh, hd, L, seed=m), list(range(m)), 0, L, ws)
+        assert bool((ws == -7.0).all()) == (m == last), m
