@@ -1057,14 +1057,18 @@ SSD_API int ssd_prefill_attention_bf16(const uint16_t* q, int64_t ldq, int M, in
       ((uintptr_t)vt_cache & 15) || ldo % 4 || ((uintptr_t)out & 7))
     return set_error(SSD_EINVAL, "prefill attention: rows [%d, %d) vs cache %lld, or misaligned operands", pos0,
                      pos0 + M, (long long)max_len);
-  // one 16-row tile per wave while that leaves at most two workgroups per CU
+  // a workgroup's four waves share one kv head's K/V when 4 divides the q heads per kv head
+  const bool shared = (heads / kv_heads) % 4 == 0;
+  // One 16-row tile per wave while that leaves at most two workgroups per CU, or one where the waves read K / V for
+  // themselves, at head_dim 128 and after a past of more than 2048 keys: two such workgroups on a CU then fetch twice
+  // what one of 32 rows does (us, one tile / two: 24 q heads on 8 kv heads, 704 rows after 1000 keys 51 / 50,
+  // 8000 292 / 208, 32000 1148 / 759; at head_dim 64 one tile stays the faster).
   const int n_hg = (heads + 3) / 4;
-  const bool small = (int64_t)((M + 15) / 16) * n_hg <= 512;
+  const int most = shared || head_dim == 64 || pos0 <= 2048 ? 512 : 256;
+  const bool small = (int64_t)((M + 15) / 16) * n_hg <= most;
   const int tok = small ? 16 : 32, n_tt = (M + tok - 1) / tok;
   const dim3 grid((unsigned)(n_tt * n_hg)), block(256);
   const float sl2 = scale * 1.4426950408889634f;
-  // a workgroup's four waves share one kv head's K/V when 4 divides the q heads per kv head
-  const bool shared = (heads / kv_heads) % 4 == 0;
 #define PF_ATT_NT(D, SH, NT)                                                                                       \
   SSD_LAUNCH((prefill_attention_kernel<D, SH, NT>), grid, block, 0, stream, (const bf16_t*)q, ldq, M, pos0, heads, \
              kv_heads, (const bf16_t*)k_cache, (const bf16_t*)vt_cache, max_len, sl2, (bf16_t*)out, ldo, n_tt)

@@ -138,3 +138,23 @@ def test_attention_rows_do_not_depend_on_the_tile(heads, kv, hd):
         out = torch.zeros(n, heads * hd, dtype=torch.bfloat16, device=DEV)
         ops.prefill_attention(q[r0:r0 + n], n, r0, heads, kv, hd, kd, vd, cap, out)
         assert torch.equal(out, ref[r0:r0 + n]), (r0, n)
+
+
+@pytest.mark.parametrize("heads,kv,hd", [(24, 8, 128), (32, 32, 128), (24, 8, 64), (32, 8, 128)])
+@pytest.mark.parametrize("pos0", [2048, 2049, 5000])
+def test_attention_rows_after_a_long_past_do_not_depend_on_the_tile(heads, kv, hd, pos0):
+    """The row count from which a wave takes 32 rows depends on the heads' sharing and on the past as well: calls on
+    both sides of each line, in rows, give a row the same bits."""
+    from ssd import ops
+
+    n_hg = heads // 4
+    m = 512 // n_hg * 16 + 16
+    cap = (pos0 + m + 63) // 64 * 64
+    q = _rand(m, heads * hd, seed=15)
+    k, v = ops.kv_tile(_rand(kv, cap, hd, seed=16), "k"), ops.kv_tile(_rand(kv, cap, hd, seed=17), "v")
+    ref = torch.zeros(m, heads * hd, dtype=torch.bfloat16, device=DEV)
+    ops.prefill_attention(q, m, pos0, heads, kv, hd, k, v, cap, ref)
+    for n in (256 // n_hg * 16, 256 // n_hg * 16 + 1, m - 16, 70):
+        out = torch.zeros(n, heads * hd, dtype=torch.bfloat16, device=DEV)
+        ops.prefill_attention(q, n, pos0, heads, kv, hd, k, v, cap, out)
+        assert torch.equal(out, ref[:n]), n
