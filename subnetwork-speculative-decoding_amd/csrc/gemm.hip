@@ -62,7 +62,9 @@ template <int CT, int NSUB, int KS, int U, int EPI, int NORM, int XR = 0>
 __global__ __launch_bounds__(64 * KS) void gemm_kernel(GemmArgs a) {
   constexpr bool XS = XR > 0;
   constexpr int XS_ROUNDS = XR;
-  constexpr int XS_AHEAD = CT * (NSUB + 2) <= 8 ? 3 : CT * (NSUB + 2) <= 18 ? 2 : 1;  // rounds of loads in registers
+  // Rounds of loads in registers, by what a round takes of them. The norm's sums need room as well: with two rounds
+  // ahead the four tiles of 33-48 rows (18) spilled to scratch (70B q/k/v, 40 rows, 40.2 us; one round 37.1).
+  constexpr int XS_AHEAD = CT * (NSUB + 2) <= 8 ? 3 : CT * (NSUB + 2) <= (NORM ? 16 : 18) ? 2 : 1;
   static_assert(!XS || KS == 8, "the staged path deals 16 k-blocks per round to 8 waves");
   __shared__ GemmSmem<KS, NSUB, CT, XS> smem;
   auto& lds = smem.g;
@@ -175,7 +177,12 @@ __global__ __launch_bounds__(64 * KS) void gemm_kernel(GemmArgs a) {
           for (int c = 0; c < CT; ++c) acc[s][c] = mfma16x16x32(bits_bf16x8(wv[r][u][s]), bits_bf16x8(xr[c]), acc[s][c]);
         if constexpr (NORM) {
 #pragma unroll
-          for (int c = 0; c < CT; ++c) ss[c] += sumsq8(xr[c]);
+          for (int c = 0; c < CT; ++c) {
+            ss[c] += sumsq8(xr[c]);
+            // shortest of all: each sum is finished before the next fragment is unpacked (70B q/k/v at 64 rows
+            // 45.0 us without, 41.7 with; at 17-32 rows it would cost 1 us)
+            if constexpr (CT * (NSUB + 2) > 18) asm volatile("" : "+v"(ss[c]));
+          }
         }
       }
       // slot (r + 1) % 2 last held round r - 1, which every wave finished before this barrier
