@@ -825,9 +825,13 @@ static GemmPlan plan_for(int N, int K) {
 // packing (a function of the shape only).
 static bool use_wide(const GemmPlan& p) { return p.nsub == 8; }
 
-// Narrow projections whose K is a whole number of 512-wide rounds take X through LDS.
-static bool staged_plan(const GemmPlan& p, int kbt) {
+// Narrow projections whose K is a whole number of 512-wide rounds take X through LDS, except where the few rows of a
+// column tile cost less to load directly than a whole staged tile does, with the norm's sums beside it: two tiles
+// a workgroup and 17 to 20 rows (us, direct / staged: N = 8192, K = 2048 8.3 / 8.9, K = 8192 21.7 / 23.1; 25 rows 9.1 / 9.1,
+// 24.7 / 24.0), at K = 2048 up to 8 rows too (7.9 / 8.1; 16 rows 8.5 / 8.4). Both give the same bits.
+static bool staged_plan(const GemmPlan& p, int kbt, int M, bool norm) {
   if (p.ks != 8) return false;
+  if (norm && p.nsub == 2 && kbt != 128 && ((M > 16 && M <= 20) || (kbt == 64 && M <= 8))) return false;
   if (kbt == 256) return p.nsub == 2 || p.nsub == 4;
   return (kbt == 64 || kbt == 128) && p.nsub <= 2;
 }
@@ -895,7 +899,7 @@ static int launch_gemm(GemmArgs a, hipStream_t s) {
     }
     const int ct = (b.M + 15) / 16;
     dim3 grid(p.tiles);
-    if (staged_plan(p, b.kb_total)) {  // x staged through LDS
+    if (staged_plan(p, b.kb_total, b.M, b.norm_eps > 0.f)) {  // x staged through LDS
 #define SSD_GEMM_XS(CT_, NS_, XR_)                                                                             \
   if (ct == CT_ && p.nsub == NS_ && b.kb_total == XR_ * 16) {                                                  \
     if (b.norm_eps > 0.f)                                                                                      \

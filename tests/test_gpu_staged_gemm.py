@@ -9,7 +9,8 @@ import torch
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
-SHAPES = [(3072, 2048), (2048, 2048), (6144, 2048), (6144, 4096), (4096, 4096), (10240, 8192), (8192, 8192)]
+SHAPES = [(3072, 2048), (2048, 2048), (6144, 2048), (6144, 4096), (4096, 4096), (10240, 8192), (8192, 8192),
+          (8192, 2048)]
 
 
 def _rand(*shape, seed, std=1.0):
@@ -27,7 +28,8 @@ def test_rows_do_not_depend_on_the_row_count(n, k, norm):
     wp = ops.pack_weight(w)
     ref = torch.zeros(80, n, dtype=torch.bfloat16, device=DEV)
     ops.gemm(x, 80, wp, n, k, ref, norm_eps=eps)
-    for m in (1, 15, 16, 17, 32, 33, 47, 49, 64, 65):
+    # (8, 9, 17, 20, 21: where calls with the norm change between staged and direct)
+    for m in (1, 8, 9, 15, 16, 17, 20, 21, 32, 33, 47, 49, 64, 65):
         out = torch.zeros(m, n, dtype=torch.bfloat16, device=DEV)
         ops.gemm(x, m, wp, n, k, out, norm_eps=eps)
         assert torch.equal(out, ref[:m]), m
