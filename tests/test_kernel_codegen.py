@@ -74,7 +74,8 @@ def _kernels(asm_text):
 
 def test_prefill_gemm_k_loop_holds_only_its_loads_and_mfmas(asm):
     found = list(_kernels(asm))
-    assert len(found) >= 6, [n for n, _, _ in found]  # {store, swiglu, q/k/v} x {row scales, none}
+    # {row scales, none} x 14 tile shapes for store and SwiGLU, 13 for q/k/v
+    assert len(found) == 2 * (14 + 14 + 13), [n for n, _, _ in found]
     for name, lines, private in found:
         assert private == 0, f"{name}: {private} bytes of scratch"
         idx = [i for i, l in enumerate(lines) if "v_mfma" in l]
