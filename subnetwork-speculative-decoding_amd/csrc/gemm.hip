@@ -45,11 +45,12 @@ struct GemmLds {
 // X staged through LDS (gemm_kernel<..., XR = K / 512>): K = 2048, 4096 or 8192 (rounds of 16 k-blocks), 8
 // waves. Each round's rows are loaded as whole 1 KiB row segments (full 128-byte lines, once per
 // workgroup) instead of each wave loading its 64-byte row pieces itself; rows are XS_ROW bytes apart so
-// the 8 lanes a b128 read serves at a time fall in different banks. A workgroup reads all of X, as many
-// bytes as its weights or more, at the ~80 GB/s of a CU's load path, which is what bounds these calls:
-// pieces of half lines cost twice. us direct / staged: 8B q/k/v at 40 and 64 rows 17.7 / 15.2 and 24.1 / 17.0,
-// o 15.0 / 11.4 and 21.5 / 13.9; 70B q/k/v at 1, 25 and 64 rows 32.7 / 28.2, 47.3 / 32.7 and 83.2 / 41.7 (with
-// four tiles a workgroup, see plan_for). Loads run three rounds ahead, fewer where registers are short.
+// the 8 lanes a b128 read serves at a time fall in different banks. A workgroup reads all of X, CT / NSUB
+// times the bytes of its weights, at the ~80 GB/s of a CU's load path, which is what bounds the calls of many
+// rows: pieces of half lines cost twice. us direct / staged: 8B q/k/v at 40 and 64 rows 17.7 / 15.2 and 24.1 /
+// 17.0, o 15.0 / 11.4 and 21.5 / 13.9; 70B q/k/v at 1, 25 and 64 rows 32.7 / 28.2, 47.3 / 32.7 and 83.2 / 41.6. The
+// last three are four tiles a workgroup against two: at one row X is a quarter of the weights' bytes, and what
+// that call gains is the one round of workgroups (see plan_for). Loads run one to three rounds ahead (XS_AHEAD).
 constexpr int XS_SLOTS = 2, XS_ROW = 16 * 64 + 16;
 
 template <int KS, int NSUB, int CT, bool XS>
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(64 * KS) void gemm_kernel(GemmArgs a) {
   constexpr bool XS = XR > 0;
   constexpr int XS_ROUNDS = XR;
   // Rounds of loads in registers, by what a round takes of them. The norm's sums need room as well: with two rounds
-  // ahead the four tiles of 33-48 rows (18) spilled to scratch (70B q/k/v, 40 rows, 40.2 us; one round 37.1).
+  // ahead the four tiles of 33-48 rows (18) spilled to scratch (70B q/k/v, 40 rows, 40.1 us; one round 37.3).
   constexpr int XS_AHEAD = CT * (NSUB + 2) <= 8 ? 3 : CT * (NSUB + 2) <= (NORM ? 16 : 18) ? 2 : 1;
   static_assert(!XS || KS == 8, "the staged path deals 16 k-blocks per round to 8 waves");
   __shared__ GemmSmem<KS, NSUB, CT, XS> smem;

@@ -46,12 +46,15 @@ __device__ __forceinline__ size_t packed_tile(int nb, int kb, int kbt, int group
 // by direct global-to-LDS loads, 16 bytes per lane: a packed W tile (one contiguous KiB), or 8 tokens
 // x 64 k of X (eight whole 128-byte lines; the eight 16-byte pieces of token r's line land at
 // positions p ^ (r & 7), so that the fragment reads, 16 tokens x one piece, hit every LDS bank
-// equally). A step is KU k-blocks of 32; W is kept in a ring of P4_WS step slots, X in a ring of XU
-// units of 64 k. Step s: wait until this wave's loads for step s + 1 have landed (those issued in
-// step s - 1 may still run) and pass one barrier; run step s's MFMAs on the fragments read one step
-// earlier, and between them -- a few after every row of MFMAs, so that neither the LDS nor the
-// address unit holds back the next MFMA -- read step s + 1's fragments and issue loads: W of step
-// s + 3, and step s's share of the X unit that replaces the oldest one. Waves' global addresses are
+// equally). A step is KU k-blocks of 32; W is kept in a ring of NS step slots, X in a ring of XU units
+// of 64 k, both loaded AHEAD = NS - 1 steps before their MFMAs. Step s: wait until this wave's loads
+// for step s + 1 have landed (those of the AHEAD - 2 steps after it may still run) and pass one barrier;
+// run step s's MFMAs on the fragments read one step earlier, and between them -- a few after every
+// row of MFMAs, so that neither the LDS nor the address unit holds back the next MFMA -- read step
+// s + 1's fragments and issue loads: W of step s + AHEAD into the slot that held step s - 1, and of X, with
+// KU = 2, that step's unit, with KU = 1 (AHEAD = 3) half of unit s / 2 + 2, which replaces unit
+// s / 2 - 1. A slot's last fragments were read in the step before its last MFMAs, which waited for
+// them before this step's barrier. Waves' global addresses are
 // scalar pointers plus one 32-bit lane offset, ring positions scalar offsets. The step body takes its
 // LDS areas as restrict pointers, which lets the compiler see that the fragment reads do not touch
 // the areas being loaded (otherwise it waits for every load in flight before each LDS read). Every
@@ -345,7 +348,7 @@ __global__ __launch_bounds__(256, OCC) void prefill_gemm4_kernel(GemmArgs a, int
       asm volatile("" : "+a"(acc[x][y]));  // here, not in each path of the k loop
     }
 
-  // Prologue: KU = 2: W and X of steps 0 .. 2. KU = 1: X unit 0 and W 0, then what step 0 and step 1
+  // Prologue: KU = 2: W and X of steps 0 .. AHEAD - 1. KU = 1: X unit 0 and W 0, then what step 0 and step 1
   // wait for one step's worth of loads after another: W 1, half of unit 1; W 2, its other half.
   auto load_x_half = [&](int h, uint32_t off) {
 #pragma unroll
@@ -398,7 +401,7 @@ __global__ __launch_bounds__(256, OCC) void prefill_gemm4_kernel(GemmArgs a, int
     for (int r = 0; r < KU * (XT + YT); ++r) p4_fetch<XT, YT, KU>(f0, rw0, nx, r);
   }
 
-  // ring positions (bytes): W slots of steps s + 1 (read) and s + 3 (loaded); X unit of step s + 1 and
+  // ring positions (bytes): W slots of steps s + 1 (read) and s + AHEAD (loaded); X unit of step s + 1 and
   // the one being loaded
   uint32_t wr = C::WSLOT, ww = C::AHEAD * C::WSLOT, xr = KU == 1 ? 0 : C::XUNIT,
            xw = (KU == 1 ? 2 : C::AHEAD) * C::XUNIT;
@@ -424,7 +427,7 @@ __global__ __launch_bounds__(256, OCC) void prefill_gemm4_kernel(GemmArgs a, int
       nx[0] = rx0 + xr + px[0];
       nx[KU - 1] = rx0 + xr + px[1];
     }
-    // KU = 1: X unit s / 2 + 2 (its first k-block is step 2 (s / 2) + 4); KU = 2: unit s + 3
+    // KU = 1: X unit s / 2 + 2 (its first k-block is step 2 (s / 2) + 4); KU = 2: unit s + AHEAD
     const bool load_w = FULL || s + C::AHEAD < n_steps;
     const bool load_x = FULL || (KU == 1 ? s - H + 4 < n_steps : s + C::AHEAD < n_steps);
     // the lane offsets pass through an empty asm statement, so that the addresses stay a scalar pointer
