@@ -41,7 +41,7 @@ CHUNK = 64       # rows per kernel launch chain (GEMM column tiles of 16 x 4)
 # prefill kernels; 100 rows 255 (two decode forwards) against 137; 32 rows 90 against 112. The prefill attention
 # has one workgroup for 16 or 32 rows of 4 heads walk all their keys, while decode attention spreads the keys
 # over the chip, so a long past turns this round: the two meet at 7900 cached tokens for 65 rows of 24 heads
-# (3B; 15000 at 1B and 8B, 33000 at 70B), 12500 for 128 (24000, 45000), 35000 for 255 (75000 and more). 100 rows after
+# (3B; 15000 at 1B and 8B, 33000 at 70B), 12500 for 128 (24000, 90000), 35000 for 255 (75000 and more). 100 rows after
 # 64000 tokens, 8B: 654 a layer through the decode kernels, 1083 through the prefill kernels.
 PREFILL_MIN = CHUNK + 1
 PREFILL_ANY_PAST = 256  # rows from which the past does not matter (four decode forwards)
